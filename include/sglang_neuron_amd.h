@@ -409,6 +409,21 @@ int sna_prefill_attention(const void *q, const void *k_cache, const void *v_cach
                           int32_t num_kv_heads, int32_t head_dim, int32_t page_size, int64_t num_blocks,
                           int32_t kv_dtype, void *stream);
 
+/* The same with the keys split where the query blocks alone do not fill the chip (short chunks after long priors): every
+ * query block's keys are cut on the device, from its lengths, into splits that fill one or two rounds of workgroups, the
+ * partials go to `workspace` (device, 16-byte aligned, at least sna_prefill_workspace_bytes bytes; it needs no
+ * initialisation) and a second launch merges them. A NULL workspace never splits. sna_prefill_workspace_bytes: 0 where
+ * the launch would not split. */
+int64_t sna_prefill_workspace_bytes(int32_t R, int32_t max_q_len, int32_t num_q_heads, int32_t num_kv_heads,
+                                    int32_t head_dim, int32_t page_size, int32_t table_width, int32_t window);
+int sna_prefill_attention_split(const void *q, const void *k_cache, const void *v_cache, const float *k_scale,
+                                const float *v_scale, const int32_t *block_table, int64_t table_stride,
+                                int32_t table_width, const int32_t *q_start, const int32_t *prior_lens, int32_t R,
+                                int32_t max_q_len, const float *sinks, float sm_scale, int32_t window, void *out,
+                                int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t page_size,
+                                int64_t num_blocks, int32_t kv_dtype, void *workspace, int64_t workspace_bytes,
+                                void *stream);
+
 /* =====================================================================================================
  * DSA indexer (the step that picks the sparse decode's positions)
  * ===================================================================================================== */

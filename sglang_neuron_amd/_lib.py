@@ -88,6 +88,9 @@ SIGNATURES = {
     "sna_lse_combine": (_I32, [_P, _P, _I32, _I64, _I32, _P, _P, _P]),
     "sna_prefill_attention": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, _P, _I32, _I32, _P, _F32, _I32, _P,
                                      _I32, _I32, _I32, _I32, _I64, _I32, _P]),
+    "sna_prefill_attention_split": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, _P, _I32, _I32, _P, _F32, _I32, _P,
+                                     _I32, _I32, _I32, _I32, _I64, _I32, _P, _I64, _P]),
+    "sna_prefill_workspace_bytes": (_I64, [_I32] * 8),
     "sna_index_key_store": (_I32, [_P, _P, _I64, _I32, _P, _I64, _P]),
     "sna_indexer_scores": (_I32, [_P, _P, _P, _P, _I64, _I32, _P, _I32, _I32, _I32, _I32, _I64, _I32, _P, _I64, _P]),
     "sna_page_items_wire_bytes": (_I64, [_P, _I32, _I64]),

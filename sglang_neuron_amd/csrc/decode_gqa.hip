@@ -74,35 +74,6 @@ __device__ __forceinline__ int32_t launched_splits(const GqaArgs& a, int32_t b, 
   return min(a.dev_split ? max(n, 1) : n, max(a.max_splits, 1));
 }
 
-template <int CTRL>
-__device__ __forceinline__ int32_t dpp_i32(int32_t v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
-}
-// Inclusive prefix sum of v over the wave's 64 lanes (lane l gets v[0] + ... + v[l]), and the wave's sum in *total
-// (uniform). Within each 16-lane row by row_shr 1, 2, 4 and 8 (a lane whose source lies before its row's start adds
-// 0: the move leaves it the old value, 0), then each row adds the sums of the rows before it, read from their last
-// lanes. VALU moves and lane reads, no LDS round trip.
-__device__ __forceinline__ int32_t wave_incl_scan_i32(int32_t v, int32_t* total) {
-  v += dpp_i32<0x111>(v);
-  v += dpp_i32<0x112>(v);
-  v += dpp_i32<0x114>(v);
-  v += dpp_i32<0x118>(v);
-  const int32_t r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31);
-  const int32_t r2 = __builtin_amdgcn_readlane(v, 47), r3 = __builtin_amdgcn_readlane(v, 63);
-  const int row = (threadIdx.x & 63) >> 4;
-  *total = r0 + r1 + r2 + r3;
-  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
-}
-// The wave's largest v (uniform) for v >= 0: running maxima within each row the same way, then the rows' last lanes.
-__device__ __forceinline__ int32_t wave_max_nonneg_i32(int32_t v) {
-  v = max(v, dpp_i32<0x111>(v));
-  v = max(v, dpp_i32<0x112>(v));
-  v = max(v, dpp_i32<0x114>(v));
-  v = max(v, dpp_i32<0x118>(v));
-  return max(max(__builtin_amdgcn_readlane(v, 15), __builtin_amdgcn_readlane(v, 31)),
-             max(__builtin_amdgcn_readlane(v, 47), __builtin_amdgcn_readlane(v, 63)));
-}
-
 // A device split's item (every lane of the calling wave gets the same values): the launch's split size st and, for
 // item w, its row b (-1 past the last item), split and the row's seq_len L, from one load of every row's length.
 // Every row has at least one split (launched_splits). The split size is the host planner's one-round rule applied

@@ -226,6 +226,18 @@ __device__ __forceinline__ void dma_global16_cached(const void* src, uint32_t ld
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src) : "memory");
 }
+// The same with a uniform 64-bit base (SGPRs) and a 32-bit byte offset per lane, so a page's address stays scalar work.
+// (s_nop 4: a base written by a lane read just before needs five wait states until a memory instruction reads it, which
+// the compiler does not add inside an asm block.)
+__device__ __forceinline__ void dma_saddr16_cached(const void* base, uint32_t voff, uint32_t lds) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
+  // (the lane read returns a signed int: each half is made unsigned before it is widened)
+  const uint32_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)base);
+  const uint32_t b_hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)base >> 32));
+  const uint64_t b = (uint64_t)b_hi << 32 | b_lo;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(voff), "s"(b)
+               : "memory");
+}
 // XCD-aware order: workgroup i of a launch runs on XCD i mod 8 (an in-bounds probe of the XCC_ID register showed it
 // for every workgroup of 256-, 512- and 1000-workgroup launches). xcd_order(i, n) deals the ids 0 .. n - 1 out so
 // that each XCD takes a contiguous run of the logical order (the first n mod 8 XCDs one item more), so consecutive
@@ -273,8 +285,10 @@ __device__ __forceinline__ f32x4_t mfma_16x16x32_bf16(const uint32_t (&a)[4], co
                                                   c, 0, 0, 0);
 }
 
-// FP8 (e4m3fn) A and B, K = 128; lane (g4, i) supplies row i of A and column i of B at the same 32 K positions, and the
-// block scale 2^(scale_b - 127) of its B block (A's scale is 1).
+// FP8 (e4m3fn) A and B, K = 128; lane (g4, i) supplies row i of A and column i of B at the same 32 K positions, and a
+// block scale 2^(scale_b - 127) of column i (A's scale is 1). Lane group g4's scale covers K block g4 of 32, which is not
+// its own 32 positions: a lane's first 16 bytes lie in block g4 / 2, its last 16 in block 2 + g4 / 2 (an in-bounds
+// probe of the builtin showed it). The same scale in every lane of a column scales the whole product.
 typedef int32_t i32x8_t __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ f32x4_t mfma_16x16x128_fp8(const uint32_t (&a)[8], const uint32_t (&b)[8], f32x4_t c,
                                                      int32_t scale_b) {
@@ -289,6 +303,25 @@ __device__ __forceinline__ f32x4_t mfma_16x16x16_bf16(const uint32_t (&a)[2], co
   u32x2_t bv = {b[0], b[1]};
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4_t, av), __builtin_bit_cast(s16x4_t, bv),
                                                     c, 0, 0, 0);
+}
+
+// The 32 x 32 shapes: the same rate in half the instructions. Lane (g2, i) = (lane / 32, lane % 32) supplies row i of A
+// and column i of B: bf16 K = 16, its 8 elements K = 8 g2 .. + 7; FP8 K = 64, 32 bytes of K at the same positions in A
+// and B (scale_b the same in every lane of a column). Element 4 q + r of the result is row 8 q + 4 g2 + r of column i.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16_t mfma_32x32x16_bf16(const uint32_t (&a)[4], const uint32_t (&b)[4], f32x16_t c) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t av = {a[0], a[1], a[2], a[3]};
+  u32x4_t bv = {b[0], b[1], b[2], b[3]};
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, av), __builtin_bit_cast(bf16x8_t, bv),
+                                                  c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16_t mfma_32x32x64_fp8(const uint32_t (&a)[8], const uint32_t (&b)[8], f32x16_t c,
+                                                      int32_t scale_b) {
+  i32x8_t av, bv;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) av[i] = (int32_t)a[i], bv[i] = (int32_t)b[i];
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, scale_b);
 }
 
 // A wave-uniform read of memory no kernel of the launch writes (block tables, index lists, seq_lens): through the
@@ -338,6 +371,11 @@ __device__ __forceinline__ float sum_across_groups(float v) {
   const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(t[0]) + __uint_as_float(t[1]);
 }
+// Over the two lanes l and l ^ 32.
+__device__ __forceinline__ float xor32_partner_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 // Reductions over the 16 lanes of each 16-lane row, in VALU data-parallel moves (no LDS round trip): quad_perm
 // [1,0,3,2] and [2,3,0,1] pair lanes within quads, row_half_mirror pairs a half-row's two quads, row_mirror the
 // row's two halves. Each step combines two lanes that then hold the same value (the operations commute), so every
@@ -362,6 +400,35 @@ __device__ __forceinline__ float row16_max(float v) {
 __device__ __forceinline__ float wave_max(float v) { return row16_max(max_across_groups(v)); }
 __device__ __forceinline__ float wave_sum(float v) { return row16_sum(sum_across_groups(v)); }
 
+template <int CTRL>
+__device__ __forceinline__ int32_t dpp_i32(int32_t v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+}
+// Inclusive prefix sum of v over the wave's 64 lanes (lane l gets v[0] + ... + v[l]), and the wave's sum in *total
+// (uniform). Within each 16-lane row by row_shr 1, 2, 4 and 8 (a lane whose source lies before its row's start adds
+// 0: the move leaves it the old value, 0), then each row adds the sums of the rows before it, read from their last
+// lanes. VALU moves and lane reads, no LDS round trip.
+__device__ __forceinline__ int32_t wave_incl_scan_i32(int32_t v, int32_t* total) {
+  v += dpp_i32<0x111>(v);
+  v += dpp_i32<0x112>(v);
+  v += dpp_i32<0x114>(v);
+  v += dpp_i32<0x118>(v);
+  const int32_t r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31);
+  const int32_t r2 = __builtin_amdgcn_readlane(v, 47), r3 = __builtin_amdgcn_readlane(v, 63);
+  const int row = (threadIdx.x & 63) >> 4;
+  *total = r0 + r1 + r2 + r3;
+  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
+// The wave's largest v (uniform) for v >= 0: running maxima within each row the same way, then the rows' last lanes.
+__device__ __forceinline__ int32_t wave_max_nonneg_i32(int32_t v) {
+  v = max(v, dpp_i32<0x111>(v));
+  v = max(v, dpp_i32<0x112>(v));
+  v = max(v, dpp_i32<0x114>(v));
+  v = max(v, dpp_i32<0x118>(v));
+  return max(max(__builtin_amdgcn_readlane(v, 15), __builtin_amdgcn_readlane(v, 31)),
+             max(__builtin_amdgcn_readlane(v, 47), __builtin_amdgcn_readlane(v, 63)));
+}
+
 // ceil(x / t) for x < 2^17 and 1 <= t < 2^17, with rt = 1 / t: the float quotient is within one of the exact one,
 // and one correction each way makes it exact.
 __device__ __forceinline__ uint32_t ceil_div_small(uint32_t x, uint32_t t, float rt) {
@@ -369,6 +436,14 @@ __device__ __forceinline__ uint32_t ceil_div_small(uint32_t x, uint32_t t, float
   if (q * t > x) --q;
   else if ((q + 1) * t <= x) ++q;
   return q + (q * t < x ? 1u : 0u);
+}
+
+// floor(x / t) for x < 2^17 and 1 <= t < 2^17, with rt = 1 / t, the same way.
+__device__ __forceinline__ uint32_t div_small(uint32_t x, uint32_t t, float rt) {
+  uint32_t q = (uint32_t)((float)x * rt);
+  if (q * t > x) --q;
+  else if ((q + 1) * t <= x) ++q;
+  return q;
 }
 
 // ---- split-K work decomposition ----

@@ -775,8 +775,8 @@ def prefill_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_table: 
     _need(block_table.dim() == 2 and block_table.shape[0] >= R and block_table.stride(1) == 1,
           "block_table must be [R, width] with unit column stride")
     q = _contig(q, "q", torch.bfloat16)
-    qs = q_start.to(torch.int32).contiguous()
-    pl = prior_lens.to(torch.int32).contiguous()
+    qs = _contig(_as(q_start, torch.int32), "q_start")
+    pl = _contig(_as(prior_lens, torch.int32), "prior_lens")
     table = block_table if block_table.dtype == torch.int32 else block_table.to(torch.int32).contiguous()
     if host_q_start is not None:
         hq = [int(x) for x in torch.as_tensor(host_q_start).reshape(-1).tolist()]
@@ -802,10 +802,14 @@ def prefill_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_table: 
     _need(out.shape == (T, H, d) and out.dtype == torch.bfloat16 and out.is_contiguous(), "out must be [T, H, d] bf16")
     if T == 0 or R == 0:
         return out
-    rc = _lib.load().sna_prefill_attention(
+    lib = _lib.load()
+    # a batch whose query blocks do not fill the chip splits its keys: partials in a workspace, merged by a second launch
+    ws_bytes = lib.sna_prefill_workspace_bytes(R, int(max_q_len), H, G, d, P, table.shape[1], int(window))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
+    rc = lib.sna_prefill_attention_split(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(ks), _ptr(vs), _ptr(table), table.stride(0), table.shape[1],
         _ptr(qs), _ptr(pl), R, int(max_q_len), _ptr(sk), float(sm_scale), int(window), _ptr(out), H, G, d, P, nb,
-        code, _stream(dev))
+        code, _ptr(ws), ws_bytes, _stream(dev))
     _lib.check(rc, "prefill_attention")
     return out
 

@@ -11,7 +11,7 @@ import torch
 from conftest import announce
 from _harness import assert_close_attn
 from oracle import attention as oatt
-from sglang_neuron_amd import ops
+from sglang_neuron_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -109,6 +109,107 @@ def test_prefill_random_shape(seed):
     bf16 pools), drawn once from fixed seeds, against the oracle."""
     cfg, window, sinks = _random_shape(seed)
     test_prefill_attention_matches_oracle(f"random-{seed}", seed, cfg, window, sinks)
+
+
+# the split's edges: one tile past the least table that splits (and too few to pay), a block's keys cut into many splits,
+# splits under a window, a group that does not divide a block's rows, chunks of unequal length (query blocks that do not
+# exist), as many blocks as a split launch takes
+SPLIT_CASES = [
+    ("seventeen-tiles", 21, dict(H=8, G=2, d=128, P=16, priors=(1025, 0), lens=(60, 5)), 0, False),
+    ("forty-tiles", 27, dict(H=8, G=2, d=128, P=16, priors=(2500, 1030), lens=(60, 5)), 0, False),
+    ("many-splits-d64", 22, dict(H=4, G=1, d=64, P=16, priors=(20000, 3), lens=(9, 70)), 0, True),
+    ("window-splits-bf16", 23, dict(H=8, G=1, d=128, P=64, priors=(9000, 700), lens=(40, 30), bf16=True), 3000, True),
+    ("group3-splits", 24, dict(H=6, G=2, d=64, P=48, priors=(2500,), lens=(43,), bf16=True), 0, False),
+    ("most-blocks", 25, dict(H=16, G=8, d=64, P=16, priors=(1600, 0), lens=(33, 1024)), 0, False),
+]
+
+
+@pytest.mark.parametrize("name,seed,cfg,window,sinks", SPLIT_CASES, ids=[c[0] for c in SPLIT_CASES])
+def test_prefill_split_edges(name, seed, cfg, window, sinks):
+    """Launches that split the keys, at the sizes where a split can go wrong; then the same call through the entry that
+    takes no workspace (which never splits): both within the attention bar of the oracle."""
+    announce(f"prefill split {name}: {cfg} window={window} sinks={sinks}")
+    q, kc, vc, ks, vs, table, q_start, priors = _case(seed, **cfg)
+    H, G, d, P, bf16 = cfg["H"], cfg["G"], cfg["d"], cfg["P"], cfg.get("bf16", False)
+    R, longest, width = len(cfg["lens"]), max(cfg["lens"]), table.shape[1]
+    sk = torch.randn(H, generator=torch.Generator().manual_seed(seed + 50)) if sinks else None
+    lib = _lib.load()
+    assert lib.sna_prefill_workspace_bytes(R, longest, H, G, d, P, width, window) > 0
+    qd, td, sd, pd = q.to(DEV), table.to(DEV), q_start.to(DEV), priors.to(DEV)
+    ksd, vsd = (None, None) if bf16 else (ks.to(DEV), vs.to(DEV))
+    skd = None if sk is None else sk.to(DEV)
+    kh, vh = (kc.cpu(), vc.cpu()) if bf16 else (kc.cpu().view(torch.uint8), vc.cpu().view(torch.uint8))
+    want = oatt.segmented_prefill(q, kh, vh, table, q_start, priors, sm_scale=d ** -0.5, k_scale=ks, v_scale=vs,
+                                  sinks=sk, window=window)
+    out = ops.prefill_attention(qd, kc, vc, td, sd, pd, max_q_len=longest, sm_scale=d ** -0.5, k_scale=ksd,
+                                v_scale=vsd, sinks=skd, window=window)
+    torch.cuda.synchronize()
+    assert_close_attn(out.cpu(), want, name)
+    whole = torch.empty_like(out)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    rc = lib.sna_prefill_attention(ptr(qd), ptr(kc), ptr(vc), ptr(ksd), ptr(vsd), ptr(td), td.stride(0), width, ptr(sd),
+                                   ptr(pd), R, longest, ptr(skd), d ** -0.5, window, ptr(whole), H, G, d, P,
+                                   kc.shape[0], _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_FP8_E4M3FN,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    torch.cuda.synchronize()
+    assert_close_attn(whole.cpu(), want, f"{name} unsplit")
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
+@pytest.mark.parametrize("prior", [70, 2500], ids=["whole", "split"])
+def test_prefill_ignores_unused_slots_and_invalid_pages(bf16, prior):
+    """NaN in every slot no query may see (page 0, the last page's tail, unused pages, a page the table marks invalid)
+    does not reach the output: against a float64 attention over the visible keys."""
+    announce(f"prefill nan slots bf16={bf16} prior={prior}")
+    H, G, d, P, n = 8, 2, 64, 16, 21
+    q, kc, vc, ks, vs, table, q_start, priors = _case(31, H=H, G=G, d=d, P=P, priors=(prior,), lens=(n,), bf16=bf16)
+    span = prior + n
+    hole = 3  # the page of keys 48 .. 63
+    table[0, hole] = -1
+    pos = torch.arange(span)
+    live = pos // P != hole
+    slots = (table[0, pos // P].to(torch.int64) * P + pos % P)[live]
+    used = torch.zeros(kc.shape[0] * P, dtype=torch.bool)
+    used[slots] = True
+    dead = (~used).reshape(kc.shape[0], 1, P, 1).to(DEV)
+    raw = torch.int16 if bf16 else torch.uint8
+    for cache in (kc, vc):
+        cache.view(raw).masked_fill_(dead, 0x7FC0 if bf16 else 0x7F)
+    one = (torch.ones(G), torch.ones(G)) if bf16 else (ks, vs)
+    k, v = ((c.cpu().float().permute(0, 2, 1, 3).reshape(-1, G, d)[slots] * s.reshape(1, G, 1)).double()
+            for c, s in zip((kc, vc), one))
+    qh = q.double().reshape(n, G, H // G, d)
+    scores = torch.stack([torch.einsum("sjd,kd->sjk", qh[:, g], k[:, g]) for g in range(G)], 1) * d ** -0.5
+    seen = pos[live][None, :] <= (prior + torch.arange(n))[:, None]
+    p = torch.softmax(scores.masked_fill(~seen[:, None, None], float("-inf")), -1)
+    want = torch.stack([torch.einsum("sjk,kd->sjd", p[:, g], v[:, g]) for g in range(G)], 1).reshape(n, H, d)
+    out = ops.prefill_attention(q.to(DEV), kc, vc, table.to(DEV), q_start.to(DEV), priors.to(DEV), max_q_len=n,
+                                sm_scale=d ** -0.5, k_scale=None if bf16 else ks.to(DEV),
+                                v_scale=None if bf16 else vs.to(DEV))
+    torch.cuda.synchronize()
+    assert_close_attn(out.cpu(), want, "nan slots")
+
+
+def test_prefill_split_workspace_refusals():
+    """A workspace smaller than the split needs, or not 16-byte aligned, is refused before any launch."""
+    q, kc, vc, ks, vs, table, q_start, priors = _case(26, H=8, G=2, d=64, P=16, priors=(1900,), lens=(20,))
+    lib = _lib.load()
+    need = lib.sna_prefill_workspace_bytes(1, 20, 8, 2, 64, 16, table.shape[1], 0)
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+    d = [t.to(DEV) for t in (q, ks, vs, table, q_start, priors)]
+    out = torch.empty_like(d[0])
+
+    def call(ptr, n):
+        return lib.sna_prefill_attention_split(
+            d[0].data_ptr(), kc.data_ptr(), vc.data_ptr(), d[1].data_ptr(), d[2].data_ptr(), d[3].data_ptr(),
+            d[3].stride(0), table.shape[1], d[4].data_ptr(), d[5].data_ptr(), 1, 20, None, 0.125, 0, out.data_ptr(), 8, 2,
+            64, 16, kc.shape[0], _lib.DTYPE_FP8_E4M3FN, ptr, n, torch.cuda.current_stream().cuda_stream)
+
+    assert need > 0 and call(ws.data_ptr(), need) == 0
+    assert call(ws.data_ptr(), need - 1) == _lib.SNA_ERR_WORKSPACE
+    assert call(ws.data_ptr() + 4, need) == _lib.SNA_ERR_INVALID_ARGUMENT
+    torch.cuda.synchronize()
 
 
 def test_segmented_attention_reference_signature():
