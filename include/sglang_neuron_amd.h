@@ -302,6 +302,23 @@ int sna_paged_decode_gqa(const void *q, const void *k_cache, const void *v_cache
                          int64_t num_blocks, int32_t cache_dtype, const sna_split_plan *plan, void *workspace,
                          int64_t workspace_bytes, void *stream);
 
+/* GQA decode of n_tokens active tokens per row (a speculative step's verify): q and out [B, n_tokens, num_q_heads,
+ * head_dim], k_new / v_new [B, n_tokens, num_kv_heads, head_dim], new_slots [B, n_tokens]; seq_lens [B] counts the prior
+ * and the active tokens, token t at position seq_len - n_tokens + t. The tokens are stored (sna_kv_store_mha on `stream`),
+ * then token t attends the row's prior keys and the active tokens 0 .. t: a workgroup's tokens in-band at their stored
+ * (dequantized) values, earlier ones from the pool, so a row's keys are read once for 16 / group tokens. A window (at
+ * least n_tokens) applies to each token. The plan: sna_plan_decode for the B rows, with window + n_tokens - 1 when there
+ * is a window and num_kv_heads * ceil(n_tokens / (16 / group)) (under a window num_kv_heads * n_tokens) workgroups an
+ * item; the workspace: sna_decode_workspace_bytes(plan, n_tokens * num_q_heads, head_dim).
+ * Replaces: _torch_attention_decode with X [B, S, Hd] (ops/attention/attention_decode.py:226-300). */
+int sna_paged_decode_gqa_multi(const void *q, void *k_cache, void *v_cache, const float *k_scale, const float *v_scale,
+                               const int32_t *block_table, int64_t table_stride, int32_t table_width,
+                               const int32_t *seq_lens, const void *k_new, const void *v_new, const int64_t *new_slots,
+                               const float *sinks, int32_t window, float sm_scale, void *out, int32_t B,
+                               int32_t n_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                               int32_t page_size, int64_t num_blocks, int32_t cache_dtype, const sna_split_plan *plan,
+                               void *workspace, int64_t workspace_bytes, void *stream);
+
 /* sna_paged_decode_gqa for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). It has no counterpart in the reference. Same arguments and results as
  * sna_paged_decode_gqa without the workspace: the split partials go to a scratch array of

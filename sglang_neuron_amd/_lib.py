@@ -79,6 +79,9 @@ SIGNATURES = {
     "sna_stream_workspace_reset": (_I32, [_P, _I64, _P]),
     "sna_paged_decode_gqa": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _I32, _F32, _P, _I32,
                                     _I32, _I32, _I32, _I32, _I64, _I32, ctypes.POINTER(SplitPlan), _P, _I64, _P]),
+    "sna_paged_decode_gqa_multi": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _I32, _F32, _P, _I32,
+                                          _I32, _I32, _I32, _I32, _I32, _I64, _I32, ctypes.POINTER(SplitPlan), _P,
+                                          _I64, _P]),
     "sna_paged_decode_gqa_noalloc": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _I32, _F32, _P,
                                             _I32, _I32, _I32, _I32, _I32, _I64, _I32, ctypes.POINTER(SplitPlan), _P]),
     "sna_mla_decode": (_I32, [_P, _P, _P, _P, _P, _I64, _I32, _P, _P, _P, _F32, _P, _I32, _I32, _I32, _I64, _I32,

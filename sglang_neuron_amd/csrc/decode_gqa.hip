@@ -23,6 +23,9 @@
 // Softmax state per head is (m, l, acc) in the log2 domain. m moves only when a tile's maximum passes it by more than
 // 8 (a factor of 256), so the accumulators are rescaled rarely. Probabilities stay <= 256, which bf16 and fp32
 // hold without loss of relative precision.
+#include <string.h>
+
+#include <algorithm>
 #include <mutex>
 
 #include "sna_device.h"
@@ -62,6 +65,11 @@ struct GqaArgs {
   float* ws_ml;  // [B, max_splits, H, 2]  reference max (log2 domain) and softmax sum
   int32_t* ws_st;  // a device split's split size, written by the decode launch for its combine (after ws_ml)
   uint16_t* out;
+  // S active tokens per row (MULTI launches; 1 otherwise): q, k_new, v_new, out and the partials have B * S rows, row
+  // b * S + t for token t of row b at position seq_len - S + t. A workgroup's 16 columns hold `tpi` tokens' group heads
+  // (one token's under a window), so a row takes `chunks` workgroups per (split, KV head). `window` then spans all S
+  // tokens' windows (token_window is one token's): every chunk of a row runs the same splits.
+  int32_t S, tpi, chunks, token_window;
 };
 
 // The splits this launch runs for row b: its entries in the plan's item map (counted on the host), or (no map: items
@@ -181,7 +189,7 @@ struct GqaTile {
   bool pvalid[2];
 };
 
-template <int D, bool FP8, int WAVES, bool FINAL, int DEPTH>
+template <int D, bool FP8, int WAVES, bool FINAL, int DEPTH, bool MULTI>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 void gqa_decode_kernel(GqaArgs a) {
   using Tile = GqaTile<D, FP8>;
@@ -199,19 +207,24 @@ void gqa_decode_kernel(GqaArgs a) {
   const int g4 = lane >> 4;
   const int li = lane & 15;
   const int g = blockIdx.y;
+  // the split item; MULTI: eight items' first chunks, then their second ones, ...: an item's chunks run on one XCD, whose
+  // L2 they share (the grid's width is a multiple of 8)
+  const int32_t item = MULTI ? (int32_t)(blockIdx.x / (8 * a.chunks) * 8 + blockIdx.x % 8) : (int32_t)blockIdx.x;
+  const int32_t chunk = MULTI ? (int32_t)(blockIdx.x / 8 % a.chunks) : 0;
+  if (MULTI && item >= a.n_work) return;
 
   int32_t b, split, st, L = 0;
   if (a.dev_split) {  // the split size and the item, from the device's lengths
-    gqa_device_item(a, (int32_t)blockIdx.x, b, split, st, L);
+    gqa_device_item(a, item, b, split, st, L);
     if (!FINAL && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *a.ws_st = st;  // for the combine
   } else {
     st = a.split_tiles;
-    if ((int32_t)blockIdx.x < a.work_n) {  // the plan's map, from the kernel arguments
-      const uint32_t e = a.work[blockIdx.x];
+    if (item < a.work_n) {  // the plan's map, from the kernel arguments
+      const uint32_t e = a.work[item];
       b = (int32_t)((e & ~kWorkLastSplit) >> 6);
       split = (int32_t)(e & 63u);
     } else {
-      locate_work<32>(a.seq_lens, a.B, a.window, st, (int32_t)blockIdx.x, b, split);
+      locate_work<32>(a.seq_lens, a.B, a.window, st, item, b, split);
     }
   }
   b = __builtin_amdgcn_readfirstlane(b);
@@ -220,14 +233,23 @@ void gqa_decode_kernel(GqaArgs a) {
   // uniform across the workgroup; a split past the plan's count (a length beyond the plan's bound) is dropped, so no
   // write leaves the workspace
   if (b < 0 || b >= a.B || split >= max(a.max_splits, 1)) return;
+  // the workgroup's columns: column c is query head g * group + c % group of token t0 + c / group (one token: heads only)
+  const int32_t t0 = MULTI ? chunk * a.tpi : 0;
+  const int32_t ntok = MULTI ? min(a.tpi, a.S - t0) : 1;
+  const int32_t cols = ntok * a.group;
+  const int32_t row0 = MULTI ? b * a.S + t0 : b;  // the first token's row in q, k_new, v_new and out
+  auto col_token = [&](int32_t c) -> int32_t { return MULTI ? c / a.group : 0; };
+  auto col_row = [&](int32_t c) -> int64_t {  // the column's (row, head) in q and out
+    const int32_t t = col_token(c);
+    return (int64_t)(row0 + t) * a.H + g * a.group + c - t * a.group;
+  };
   // Query operand: in step s lane (g4, li) holds head li's 8 elements from dim CE (4 c + g4) + w, with CE the
   // elements of a 16-byte cache chunk and 8 s = CE c + w: the dims of the key bytes it feeds in that step.
   constexpr int CE = 16 / ESZ;
   uint32_t qv[STEPS][4];
   {
-    const bool live = li < a.group;
-    const int32_t h = g * a.group + (live ? li : 0);
-    const uint16_t* qp = a.q + ((int64_t)b * a.H + h) * D;
+    const bool live = li < cols;
+    const uint16_t* qp = a.q + (MULTI ? col_row(live ? li : 0) : (int64_t)b * a.H + g * a.group + (live ? li : 0)) * D;
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
       const int dim = CE * (4 * (8 * s / CE) + g4) + (8 * s) % CE;
@@ -252,7 +274,7 @@ void gqa_decode_kernel(GqaArgs a) {
   const float vscale = (FP8 && a.mul_scale) ? 1.0f / vstored : vstored;
   // the group's sink logits (final outputs only), loaded with the prologue's loads: read after the tile loop, a load
   // there would add a memory round trip to the end of every workgroup
-  const float sink_pre = (FINAL && a.sinks && tid < a.group) ? a.sinks[g * a.group + tid] : 0.0f;
+  const float sink_pre = (FINAL && a.sinks && tid < cols) ? a.sinks[g * a.group + tid - col_token(tid) * a.group] : 0.0f;
   const float qk_scale = a.sm_scale * kscale * kLog2e;
   const int64_t head_stride = (int64_t)a.P * D * ESZ;  // bytes of one (page, head) block
   const int32_t* trow = a.table + (int64_t)b * a.table_stride;
@@ -277,8 +299,16 @@ void gqa_decode_kernel(GqaArgs a) {
     }
   }
   L = __builtin_amdgcn_readfirstlane(len_v);
-  const KeyRange kr = key_range(L, a.window);
-  const int32_t t_first = kr.lo / 32 + split * st;
+  // the keys the workgroup reads from the pool, visible to all its columns: MULTI the prior ones of the chunk's first
+  // token (the chunk's own tokens are attended in-band; under a window a chunk is one token), a part of the range
+  // [krow.lo, krow.hi) that the row's splits divide
+  const KeyRange krow = key_range(L, a.window);
+  KeyRange kr = krow;
+  if constexpr (MULTI) {
+    kr.hi = max(L - a.S + t0, 0);
+    kr.lo = a.token_window > 0 ? max(0, kr.hi + 1 - a.token_window) : 0;
+  }
+  const int32_t t_first = krow.lo / 32 + split * st;
   const int32_t t_last = min(t_first + st, (kr.hi + 31) / 32);
   bool pre = true;
   if (!early) {
@@ -419,17 +449,31 @@ void gqa_decode_kernel(GqaArgs a) {
   // the items were located from seq_lens, up to the plan's split count. So the own token is attended and stored even
   // when the device's length disagrees with the plan's.
   // (with a map the item's own flag says it, from the entry already loaded)
-  const bool own = (int32_t)blockIdx.x < a.work_n ? (a.work[blockIdx.x] & kWorkLastSplit) != 0
-                                                   : split == launched_splits(a, b, L, st) - 1;  // uniform
+  const bool own = item < a.work_n ? (a.work[item] & kWorkLastSplit) != 0
+                                   : split == launched_splits(a, b, L, st) - 1;  // uniform
   constexpr int OWN_J = (16 + WAVES - 1) / WAVES;  // query heads per wave in the own token's score
-  uint32_t own_kb = 0, own_vb = 0;
+  constexpr int OWN_T = MULTI ? 16 : 1;                       // the most tokens of a workgroup
+  constexpr int OWN_E = (OWN_T * D + 64 * WAVES - 1) / (64 * WAVES);  // their elements per thread
+  uint32_t own_kb[OWN_E] = {}, own_vb[OWN_E] = {};
   int64_t own_dst = -1;
   float own_q[OWN_J][D / 64];
   if (own) {
-    if (tid < D) {
+    if constexpr (MULTI) {
+      // (the tokens were stored before the launch, which reads the earlier ones from the pool)
+#pragma unroll
+      for (int i = 0; i < OWN_E; ++i) {
+        const int e = tid + 64 * WAVES * i;
+        own_kb[i] = own_vb[i] = 0;
+        if (e < ntok * D) {
+          const int64_t src = ((int64_t)(row0 + e / D) * a.G + g) * D + e % D;
+          own_kb[i] = a.k_new[src];
+          own_vb[i] = a.v_new[src];
+        }
+      }
+    } else if (tid < D) {
       const int64_t src = ((int64_t)b * a.G + g) * D + tid;
-      own_kb = a.k_new[src];
-      own_vb = a.v_new[src];
+      own_kb[0] = a.k_new[src];
+      own_vb[0] = a.v_new[src];
       if (a.new_slots) {
         const int64_t slot = redirect_slot(a.new_slots[b], a.num_blocks * a.P);
         own_dst = (((slot / a.P) * a.G + g) * a.P + slot % a.P) * D + tid;
@@ -438,7 +482,8 @@ void gqa_decode_kernel(GqaArgs a) {
 #pragma unroll
     for (int jj = 0; jj < OWN_J; ++jj) {
       const int j = wave + WAVES * jj;
-      const uint16_t* qp = a.q + ((int64_t)b * a.H + g * a.group + min(j, a.group - 1)) * D;
+      const uint16_t* qp = a.q + (MULTI ? col_row(min(j, cols - 1))
+                                        : (int64_t)b * a.H + g * a.group + min(j, a.group - 1)) * D;
 #pragma unroll
       for (int v = 0; v < D / 64; ++v) own_q[jj][v] = bf16_bits_to_f32(qp[lane + 64 * v]);
     }
@@ -469,10 +514,13 @@ void gqa_decode_kernel(GqaArgs a) {
   }
 
   // ---- the step's own token (operands loaded before the tile loop) ----
-  __shared__ float sm_kn[D], sm_vn[D], sm_sn[16];
+  __shared__ float sm_kn[OWN_T * D], sm_vn[OWN_T * D], sm_sn[16 * OWN_T];
   if (own) {
-    if (tid < D) {
-      const uint32_t kb = own_kb, vb = own_vb;
+#pragma unroll
+    for (int i = 0; i < OWN_E; ++i) {
+      const int e = tid + 64 * WAVES * i;
+      if (e >= (MULTI ? ntok * D : D)) break;
+      const uint32_t kb = own_kb[i], vb = own_vb[i];
       const int64_t dst = own_dst;
       float kd, vd;
       if constexpr (FP8) {
@@ -492,26 +540,28 @@ void gqa_decode_kernel(GqaArgs a) {
           reinterpret_cast<uint16_t*>(a.v_cache)[dst] = (uint16_t)vb;
         }
       }
-      sm_kn[tid] = kd;
-      sm_vn[tid] = vd;
+      sm_kn[e] = kd;
+      sm_vn[e] = vd;
     }
     __syncthreads();
 #pragma unroll
     for (int jj = 0; jj < OWN_J; ++jj) {
       const int j = wave + WAVES * jj;  // uniform
-      if (j >= a.group) break;
-      float s = 0.0f;
+      if (j >= cols) break;
+      for (int u = 0; u <= col_token(j); ++u) {  // the workgroup's tokens up to the column's own
+        float s = 0.0f;
 #pragma unroll
-      for (int v = 0; v < D / 64; ++v) s += own_q[jj][v] * sm_kn[lane + 64 * v];
-      s = wave_sum(s);
-      if (lane == 0) sm_sn[j] = s * a.sm_scale * kLog2e;
+        for (int v = 0; v < D / 64; ++v) s += own_q[jj][v] * sm_kn[u * D + lane + 64 * v];
+        s = wave_sum(s);
+        if (lane == 0) sm_sn[j * OWN_T + u] = s * a.sm_scale * kLog2e;
+      }
     }
   }
 
   // ---- merge the waves (and the own token) in LDS; write the output or this split's partial ----
   __shared__ float sm_o[WAVES][16][D + 1];
   __shared__ float sm_sink[16];
-  if (FINAL && tid < a.group) sm_sink[tid] = sink_pre;
+  if (FINAL && tid < cols) sm_sink[tid] = sink_pre;
   __shared__ float sm_m[WAVES][16];
   __shared__ float sm_l[WAVES][16];
   const float l_tot = sum_across_groups(l_run);
@@ -525,10 +575,12 @@ void gqa_decode_kernel(GqaArgs a) {
   }
   __syncthreads();
   const int32_t S = a.max_splits;
-  for (int idx = tid; idx < a.group * D; idx += 64 * WAVES) {
+  for (int idx = tid; idx < cols * D; idx += 64 * WAVES) {
     const int j = idx / D, d = idx % D;
-    const int32_t h = g * a.group + j;
-    float M = own ? sm_sn[j] : -INFINITY;
+    const int32_t t = col_token(j), h = g * a.group + j - t * a.group;
+    float M = -INFINITY;
+    if (own)
+      for (int u = 0; u <= t; ++u) M = fmaxf(M, sm_sn[j * OWN_T + u]);
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) M = fmaxf(M, sm_m[w][j]);
     float o = 0.0f, l = 0.0f;
@@ -540,15 +592,17 @@ void gqa_decode_kernel(GqaArgs a) {
     }
     o *= vscale;
     if (own) {
-      const float e = __builtin_amdgcn_exp2f(sm_sn[j] - M);
-      o += e * sm_vn[d];
-      l += e;
+      for (int u = 0; u <= t; ++u) {
+        const float e = __builtin_amdgcn_exp2f(sm_sn[j * OWN_T + u] - M);
+        o += e * sm_vn[u * D + d];
+        l += e;
+      }
     }
     if constexpr (FINAL) {
       if (a.sinks) l += __builtin_amdgcn_exp2f(sm_sink[j] * kLog2e - M);
-      a.out[((int64_t)b * a.H + h) * D + d] = (uint16_t)f32_to_bf16_bits(o / l);
+      a.out[((int64_t)(row0 + t) * a.H + h) * D + d] = (uint16_t)f32_to_bf16_bits(o / l);
     } else {
-      const int64_t row = ((int64_t)b * S + split) * a.H + h;
+      const int64_t row = ((int64_t)(row0 + t) * S + split) * a.H + h;
       a.ws_o[row * D + d] = o;
       if (d == 0) {
         a.ws_ml[row * 2] = M;
@@ -581,7 +635,8 @@ __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
     for (int v = 0; v < V; ++v) x[k][v] = k < S ? ob[k * sstride + v] : 0.0f;
   float2 ml = make_float2(-INFINITY, 0.0f);
   if (lane < S) ml = *reinterpret_cast<const float2*>(a.ws_ml + (row0 + (int64_t)lane * a.H) * 2);
-  const int32_t n = min(launched_splits(a, b, ld_const(a.seq_lens + b), a.dev_split ? *a.ws_st : a.split_tiles), S);
+  const int32_t br = a.S == 1 ? b : b / a.S;  // the row of seq_lens (S tokens a row)
+  const int32_t n = min(launched_splits(a, br, ld_const(a.seq_lens + br), a.dev_split ? *a.ws_st : a.split_tiles), S);
   if (n == 0) return;  // a row with no prior key: the lone-token kernel writes it
   const float m = lane < n ? ml.x : -INFINITY, l = lane < n ? ml.y : 0.0f;
   const float sink = a.sinks ? a.sinks[h] * kLog2e : -INFINITY;
@@ -618,7 +673,8 @@ template <int D, bool FP8>
 __global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgs a) {
   const int b = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
   // any split size counts the row's splits as nonzero iff it has a prior key
-  if (launched_splits(a, b, a.seq_lens[b], a.split_tiles) > 0) return;
+  const int32_t br = a.S == 1 ? b : b / a.S;  // (S tokens a row)
+  if (launched_splits(a, br, a.seq_lens[br], a.split_tiles) > 0) return;
   __shared__ float sm_kn[D], sm_vn[D];
   const float kstored = FP8 ? a.k_scale[g] : 1.0f, vstored = FP8 ? a.v_scale[g] : 1.0f;
   const float kscale = (FP8 && a.mul_scale) ? 1.0f / kstored : kstored;
@@ -669,25 +725,35 @@ __global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgs a) {
   }
 }
 
-template <int D, bool FP8>
+template <int D, bool FP8, bool MULTI>
 static void launch_gqa(const GqaArgs& a, bool any_lone, hipStream_t s) {
   if (a.n_work > 0) {
-    const dim3 grid(a.n_work, a.G);
+    const dim3 grid(MULTI ? (a.n_work + 7) / 8 * 8 * a.chunks : a.n_work, a.G);
     // two register tiles per wave whatever the plan's shape (rings of 3 and 4 measured 1% and 2% slower on the cfg2
     // and cfg4 batches: fewer loads outstanding per wave stream faster). Splits of 5 to 64 tiles run on 8 waves, so
     // a wave walks half as many tiles one after the other (cfg4-swa's 5-tile rows 7.98 -> 6.45 us, cfg4's 48-tile
-    // splits 24.9 -> 24.3, cfg1's 8-tile splits 12.3 -> 12.1); cfg2's whole 128-tile rows stay on 4 (91 against 94).
-    const bool eight = a.split_tiles > 4 && a.split_tiles <= 64;
+    // splits 24.9 -> 24.3, cfg1's 8-tile splits 12.3 -> 12.1), where a CU holds two such workgroups (head dim 64) or
+    // the launch has one a CU: at head dim 128 their registers leave room for one, so a plan's one round would run as
+    // two (16 rows of 500-2000 keys, 32 / 8 heads, FP8: 21.1 us on 8 waves, 16.8 on 4; one row of 32000 25.2 and 21.9;
+    // 16 rows of 1000-8000 35.8 and 32.7). cfg2's whole 128-tile rows run on 4 (91 against 94).
+    const bool eight = a.split_tiles > 4 && a.split_tiles <= 64 &&
+                       (D == 64 || (int64_t)a.n_work * a.chunks * a.G <= 256);
     if (a.max_splits <= 1) {
-      if (eight) hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 8, true, 2>), grid, dim3(512), 0, s, a);
-      else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, true, 2>), grid, dim3(256), 0, s, a);
+      if (eight) hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 8, true, 2, MULTI>), grid, dim3(512), 0, s, a);
+      else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, true, 2, MULTI>), grid, dim3(256), 0, s, a);
     } else {
-      if (eight) hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 8, false, 2>), grid, dim3(512), 0, s, a);
-      else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, false, 2>), grid, dim3(256), 0, s, a);
+      if (eight) hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 8, false, 2, MULTI>), grid, dim3(512), 0, s, a);
+      else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, false, 2, MULTI>), grid, dim3(256), 0, s, a);
     }
   }
-  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.B, a.H), dim3(64), 0, s, a);
-  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8>), dim3(a.B, a.G), dim3(128), 0, s, a);
+  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.B * a.S, a.H), dim3(64), 0, s, a);
+  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8>), dim3(a.B * a.S, a.G), dim3(128), 0, s, a);
+}
+
+template <int D, bool FP8>
+static void launch_gqa_tokens(const GqaArgs& a, bool any_lone, hipStream_t s) {
+  if (a.S > 1) launch_gqa<D, FP8, true>(a, any_lone, s);
+  else launch_gqa<D, FP8, false>(a, any_lone, s);
 }
 
 }  // namespace sna
@@ -708,7 +774,8 @@ int decode_gqa(const char* what, const void* q, const void* k_cache, const void*
                const int32_t* seq_lens, const void* k_new, const void* v_new, const int64_t* new_slots,
                const float* sinks, int32_t window, float sm_scale, void* out, int32_t B, int32_t num_q_heads,
                int32_t num_kv_heads, int32_t head_dim, int32_t page_size, int64_t num_blocks, int32_t cache_dtype,
-               const sna_split_plan* plan, void* workspace, int64_t workspace_bytes, void* stream) {
+               const sna_split_plan* plan, void* workspace, int64_t workspace_bytes, void* stream, int32_t S = 1,
+               bool store_first = false) {
   if (B < 0 || num_q_heads < 1 || num_kv_heads < 1 || num_q_heads % num_kv_heads)
     return fail(SNA_ERR_INVALID_ARGUMENT, "%s: bad head counts (q %d, kv %d)", what, num_q_heads, num_kv_heads);
   const int32_t group = num_q_heads / num_kv_heads;
@@ -733,7 +800,9 @@ int decode_gqa(const char* what, const void* q, const void* k_cache, const void*
                 kGqaDevSplitRows, B);
   if (B == 0) return SNA_OK;
   const bool fp8 = cache_dtype != SNA_DTYPE_BF16;
-  const int64_t need = sna_decode_workspace_bytes(plan, num_q_heads, head_dim);
+  if ((int64_t)B * S > INT32_MAX / 64 || (int64_t)num_q_heads * S > INT32_MAX)
+    return fail(SNA_ERR_INVALID_ARGUMENT, "%s: %d rows of %d tokens exceed the grid", what, B, S);
+  const int64_t need = sna_decode_workspace_bytes(plan, num_q_heads * S, head_dim);
   if (!q || !k_cache || !v_cache || !block_table || !seq_lens || !k_new || !v_new || !out ||
       (fp8 && (!k_scale || !v_scale)) || (need > 0 && !workspace))
     return fail(SNA_ERR_INVALID_ARGUMENT, "%s: null pointer", what);
@@ -765,33 +834,45 @@ int decode_gqa(const char* what, const void* q, const void* k_cache, const void*
   a.group = group;
   a.P = page_size;
   a.num_blocks = num_blocks;
-  a.window = window;
+  a.S = S;
+  a.tpi = window > 0 ? 1 : std::min(16 / group, S);
+  a.chunks = (S + a.tpi - 1) / a.tpi;
+  a.token_window = window;
+  a.window = window > 0 ? window + S - 1 : 0;
   a.sm_scale = sm_scale;
   a.split_tiles = plan->split_tiles;
   a.dev_split = plan->device_split;
   a.n_work = plan->n_work;
   a.max_splits = plan->max_splits;
   a.work_n = plan->work_n;
-  for (int32_t i = 0; i < plan->work_n; ++i) a.work[i] = plan->work[i];
+  // a row with no prior key has no split: the lone-token pass writes it (launched unless the plan rules it out)
+  const bool any_lone = !plan->device_split && plan->empty_rows != 0;
   if (plan->work_n > 0) {
-    for (int32_t r = 0; r < B; ++r) a.row_splits[r] = 0;
-    for (int32_t i = 0; i < plan->work_n; ++i) ++a.row_splits[(plan->work[i] & ~kWorkLastSplit) >> 6];
+    memcpy(a.work, plan->work, plan->work_n * sizeof(a.work[0]));
+    if (plan->max_splits > 1 || any_lone) {  // read by the combine and lone-token passes only
+      memset(a.row_splits, 0, B);
+      for (int32_t i = 0; i < plan->work_n; ++i) ++a.row_splits[(plan->work[i] & ~kWorkLastSplit) >> 6];
+    }
   }
   float* ws = (float*)workspace;
   a.ws_o = need > 0 ? ws : nullptr;
-  a.ws_ml = need > 0 ? ws + (int64_t)B * plan->max_splits * num_q_heads * head_dim : nullptr;
-  a.ws_st = need > 0 ? (int32_t*)(a.ws_ml + (int64_t)B * plan->max_splits * num_q_heads * 2) : nullptr;
+  a.ws_ml = need > 0 ? ws + (int64_t)B * S * plan->max_splits * num_q_heads * head_dim : nullptr;
+  a.ws_st = need > 0 ? (int32_t*)(a.ws_ml + (int64_t)B * S * plan->max_splits * num_q_heads * 2) : nullptr;
   a.out = (uint16_t*)out;
-  // a row with no prior key has no split: the lone-token pass writes it (launched unless the plan rules it out)
-  const bool any_lone = !plan->device_split && plan->empty_rows != 0;
 
   hipStream_t s = (hipStream_t)stream;
+  if (store_first) {
+    if (const int rc = sna_kv_store_mha(k_new, v_new, new_slots, (int64_t)B * S, k_scale, v_scale, a.k_cache,
+                                        a.v_cache, num_blocks, num_kv_heads, page_size, head_dim, cache_dtype, stream))
+      return rc;
+    a.new_slots = nullptr;
+  }
   if (head_dim == 128) {
-    if (fp8) launch_gqa<128, true>(a, any_lone, s);
-    else launch_gqa<128, false>(a, any_lone, s);
+    if (fp8) launch_gqa_tokens<128, true>(a, any_lone, s);
+    else launch_gqa_tokens<128, false>(a, any_lone, s);
   } else {
-    if (fp8) launch_gqa<64, true>(a, any_lone, s);
-    else launch_gqa<64, false>(a, any_lone, s);
+    if (fp8) launch_gqa_tokens<64, true>(a, any_lone, s);
+    else launch_gqa_tokens<64, false>(a, any_lone, s);
   }
   return check_launch(what);
 }
@@ -858,4 +939,24 @@ extern "C" int sna_paged_decode_gqa_noalloc(const void* q, const void* k_cache, 
   return decode_gqa(what, q, k_cache, v_cache, k_scale, v_scale, block_table, table_stride, table_width, seq_lens,
                     k_new, v_new, new_slots, sinks, window, sm_scale, out, B, num_q_heads, num_kv_heads, head_dim,
                     page_size, num_blocks, cache_dtype, plan, ws, kScratchBytes, stream);
+}
+
+extern "C" int sna_paged_decode_gqa_multi(const void* q, void* k_cache, void* v_cache, const float* k_scale,
+                                          const float* v_scale, const int32_t* block_table, int64_t table_stride,
+                                          int32_t table_width, const int32_t* seq_lens, const void* k_new,
+                                          const void* v_new, const int64_t* new_slots, const float* sinks,
+                                          int32_t window, float sm_scale, void* out, int32_t B, int32_t n_tokens,
+                                          int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                          int32_t page_size, int64_t num_blocks, int32_t cache_dtype,
+                                          const sna_split_plan* plan, void* workspace, int64_t workspace_bytes,
+                                          void* stream) {
+  ApiGuard guard;
+  const char* what = "paged_decode_gqa_multi";
+  if (n_tokens < 1 || (window > 0 && n_tokens > window))
+    return fail(SNA_ERR_INVALID_ARGUMENT, "%s: %d active tokens (at least one, and no more than a window of %d)", what,
+                n_tokens, window);
+  if (!new_slots && B > 0) return fail(SNA_ERR_INVALID_ARGUMENT, "%s: null pointer", what);
+  return decode_gqa(what, q, k_cache, v_cache, k_scale, v_scale, block_table, table_stride, table_width, seq_lens,
+                    k_new, v_new, new_slots, sinks, window, sm_scale, out, B, num_q_heads, num_kv_heads, head_dim,
+                    page_size, num_blocks, cache_dtype, plan, workspace, workspace_bytes, stream, n_tokens, true);
 }

@@ -543,15 +543,19 @@ def paged_decode_gqa_multi(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     new_slots [B, S], seq_lens [B] counting the prior and the S tokens (token j at position L - S + j). Token j
     attends the row's prior and active tokens 0 .. j. Returns [B, S, H, d] bf16.
 
-    The S tokens are stored first (kv_store_mha), then each (row, token) decodes as a row of its own whose length
-    ends at that token: its earlier active tokens are then pool keys holding the bytes the store wrote, which are the
-    values the reference attends in its last S slots (dequantized FP8 or bf16), so this is the reference's triu mask
-    over the active slots. A window must hold the S tokens (S <= window), as the reference's mask does not window
-    them. Stands in for _torch_attention_decode with X [B, S, Hd] (ops/attention/attention_decode.py:226-300)."""
+    The S tokens are stored first, then one launch decodes every row (sna_paged_decode_gqa_multi): 16 / group tokens
+    share a workgroup's columns, so a row's keys are read once for them; those tokens attend one another in-band at the
+    values the store wrote (dequantized FP8 or bf16) and earlier active tokens from the pool, which is the reference's
+    triu mask over its last S slots. A window must hold the S tokens (S <= window), as the reference's mask does not
+    window them. Stands in for _torch_attention_decode with X [B, S, Hd] (ops/attention/attention_decode.py:226-300)."""
     dev = _on_gpu(q, k_cache, v_cache, block_table, seq_lens, k_new, v_new, new_slots, k_scale, v_scale, sinks)
     _need(q.dim() == 4, lambda: f"q must be [B, S, H, d], got {tuple(q.shape)}")
     B, S, H, d = q.shape
-    nb, G, P, _ = k_cache.shape
+    nb, G, P, dk = k_cache.shape
+    _need(dk == d and v_cache.shape == k_cache.shape and v_cache.dtype == k_cache.dtype,
+          lambda: f"caches {tuple(k_cache.shape)} / {tuple(v_cache.shape)} do not match q's head_dim {d}")
+    _need(k_cache.is_contiguous() and v_cache.is_contiguous(), "caches must be contiguous")
+    _need(H % G == 0, lambda: f"{H} query heads over {G} KV heads")
     _need(k_new.shape == (B, S, G, d) and v_new.shape == (B, S, G, d),
           lambda: f"k_new / v_new must be [{B}, {S}, {G}, {d}]")
     _need(new_slots.numel() == B * S, lambda: f"new_slots must be [{B}, {S}]")
@@ -559,17 +563,38 @@ def paged_decode_gqa_multi(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     hl = _host_lens(seq_lens, host_seq_lens)
     if hl is not None:
         _need(int(hl.min()) >= S if B else True, lambda: f"a row holds its {S} active tokens: seq_lens >= {S}")
-    kv_store_mha(k_new.reshape(B * S, G, d), v_new.reshape(B * S, G, d), new_slots.reshape(-1), k_cache, v_cache,
-                 k_scale, v_scale, scales_multiply=scales_multiply)
-    j = torch.arange(S, device=dev, dtype=torch.int32)
-    lens = (seq_lens.reshape(B, 1).to(torch.int32) - S + 1 + j).reshape(-1)
-    rows = torch.arange(B, device=dev).repeat_interleave(S)
-    table = block_table.index_select(0, rows)
-    host_rows = None if hl is None else (hl.reshape(B, 1).to(torch.int32) - S + 1 + j.cpu()).reshape(-1)
-    out = paged_decode_gqa(q.reshape(B * S, H, d), k_cache, v_cache, table, lens, k_new.reshape(B * S, G, d),
-                           v_new.reshape(B * S, G, d), sm_scale=sm_scale, k_scale=k_scale, v_scale=v_scale,
-                           sinks=sinks, window=window, scales_multiply=scales_multiply, host_seq_lens=host_rows)
-    return out.reshape(B, S, H, d)
+    code = cache_dtype_code(k_cache.dtype, scales_multiply)
+    q = _contig(q, "q", torch.bfloat16)
+    k_new = _contig(k_new, "k_new", torch.bfloat16)
+    v_new = _contig(v_new, "v_new", torch.bfloat16)
+    slots = _contig(_as(new_slots.reshape(-1), torch.int64), "new_slots")
+    _need(block_table.dim() == 2 and block_table.shape[0] == B, lambda: f"block_table must be [{B}, width]")
+    table = _as(block_table, torch.int32)
+    table = table if table.stride(1) == 1 else table.contiguous()
+    lens = _contig(_as(seq_lens.reshape(-1), torch.int32), "seq_lens")
+    _need(lens.numel() == B, lambda: f"{lens.numel()} seq_lens for {B} rows")
+    if code != _lib.DTYPE_BF16:
+        _need(k_scale is not None and v_scale is not None, "an FP8 cache needs k_scale and v_scale")
+        k_scale = _contig(_as(k_scale.reshape(-1), torch.float32), "k_scale")
+        v_scale = _contig(_as(v_scale.reshape(-1), torch.float32), "v_scale")
+        _need(k_scale.numel() == G and v_scale.numel() == G, "one k/v scale per KV head")
+    if sinks is not None:
+        sinks = _contig(_as(sinks.reshape(-1), torch.float32), "sinks")
+        _need(sinks.numel() == H, lambda: f"{sinks.numel()} sinks for {H} heads")
+    out = torch.empty(B, S, H, d, dtype=torch.bfloat16, device=dev)
+    if out.numel() == 0:
+        return out
+    # a row's workgroups per (split, KV head): 16 / group tokens each, one under a window
+    chunks = S if window > 0 else -(-S // max(1, 16 // (H // G)))
+    plan = plan_decode(_lib.KIND_GQA, B, host_seq_lens=hl, max_seq_len=table.shape[1] * P,
+                       window=window + S - 1 if window > 0 else 0, ctas_per_item=G * chunks, num_cus=_num_cus(dev))
+    ws = torch.empty(max(workspace_bytes(plan, H * S, d), 16), dtype=torch.uint8, device=dev)
+    rc = _lib.load().sna_paged_decode_gqa_multi(
+        _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), _ptr(table), table.stride(0),
+        table.shape[1], _ptr(lens), _ptr(k_new), _ptr(v_new), _ptr(slots), _ptr(sinks), int(window), float(sm_scale),
+        _ptr(out), B, S, H, G, d, P, nb, code, plan, _ptr(ws), ws.numel(), _stream(dev))
+    _lib.check(rc, "paged_decode_gqa_multi")
+    return out
 
 
 def prepare_mla_decode(ql_nope: Tensor, q_pe: Tensor, cache: Tensor, row_scale: Optional[Tensor], block_table: Tensor,

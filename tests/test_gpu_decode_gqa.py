@@ -171,7 +171,16 @@ def test_gqa_device_split_plan_matches_oracle(name, cfg, over, bound):
 MULTI = [("cfg4-s4", 4, {"B": 8, "lens": (100, 3000)}, 4),                  # GPT-OSS multipliers, sinks
          ("cfg4-swa-s8", 4, {"B": 6, "lens": (2, 900), "window": 128}, 8),
          ("cfg2-s3", 2, {"B": 4, "lens": (40, 1000)}, 3),
-         ("cfg1-bf16-s2", 1, {"B": 3, "lens": (30, 400)}, 2)]
+         ("cfg1-bf16-s2", 1, {"B": 3, "lens": (30, 400)}, 2),
+         # the columns' edges: tokens past one workgroup's 16 columns (groups 1, 4, 8 and 3), one token a workgroup
+         # (group 16), a window shorter than the tokens' chunk would be, rows of only their active tokens
+         ("group1-s17", 1, {"B": 2, "H": 2, "G": 2, "lens": (20, 200)}, 17),
+         ("group4-s9", 2, {"B": 3, "H": 8, "G": 2, "lens": (9, 700)}, 9),
+         ("group8-s3-long", 4, {"B": 2, "lens": (5000, 6000)}, 3),
+         ("group3-s6", 2, {"B": 2, "H": 6, "G": 2, "d": 64, "lens": (6, 90)}, 6),
+         ("group16-s2", 1, {"B": 2, "H": 16, "G": 1, "lens": (40, 300)}, 2),
+         ("window-s5", 2, {"B": 3, "lens": (5, 400), "window": 33}, 5),
+         ("one-token", 1, {"B": 3, "lens": (1, 100)}, 1)]
 
 
 @pytest.mark.parametrize("name,cfg,over,S", MULTI, ids=[m[0] for m in MULTI])
@@ -227,3 +236,63 @@ def test_gqa_multi_token_decode_matches_oracle(name, cfg, over, S):
     assert_close_attn(out, want, name)
     assert torch.equal(cache_bytes(kc), cache_bytes(kc_o)), "K pool differs"
     assert torch.equal(cache_bytes(vc), cache_bytes(vc_o)), "V pool differs"
+
+
+def _multi_inputs(seed, B, S, H, G, d, P, lens):
+    g = torch.Generator().manual_seed(seed)
+    pages = -(-max(lens) // P)
+    nb = B * pages + 1
+    table = (torch.randperm(nb - 1, generator=g) + 1).to(torch.int32).reshape(B, pages)
+    kc, vc = (torch.randn(nb, G, P, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    q, kn, vn = (torch.randn(B, S, n, d, generator=g).to(torch.bfloat16) for n in (H, G, G))
+    slots = torch.tensor([[int(table[b, max(L - S + j, 0) // P]) * P + max(L - S + j, 0) % P for j in range(S)]
+                          for b, L in enumerate(lens)])
+    return q, kc, vc, table, kn, vn, slots
+
+
+@pytest.mark.parametrize("window", [0, 40])
+def test_gqa_multi_later_tokens_nan_stays_theirs(window):
+    """A NaN in the last active token's K and V reaches no earlier token's output (their keys end before it), whether
+    the tokens share a workgroup's columns or not."""
+    from sglang_neuron_amd import ops
+
+    B, S, H, G, d, P = 2, 4, 8, 2, 64, 16
+    lens = [90, 37]
+    q, kc, vc, table, kn, vn, slots = _multi_inputs(5, B, S, H, G, d, P, lens)
+    announce(f"gqa multi nan window={window}")
+
+    def run(kn, vn):
+        return ops.paged_decode_gqa_multi(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(),
+                                          torch.tensor(lens, dtype=torch.int32).cuda(), kn.cuda(), vn.cuda(),
+                                          sm_scale=0.125, new_slots=slots.cuda(), window=window, host_seq_lens=lens).cpu()
+
+    clean = run(kn, vn)
+    kb, vb = kn.clone(), vn.clone()
+    kb[:, -1], vb[:, -1] = float("nan"), float("nan")
+    out = run(kb, vb)
+    assert torch.equal(out[:, :-1], clean[:, :-1]) and bool(torch.isfinite(clean).all())
+    assert bool(torch.isnan(out[:, -1]).all())
+
+
+def test_gqa_multi_device_lengths_and_padding_rows():
+    """Without host lengths (a bound plan, split on the device) the outputs are those of an exact plan within a bf16
+    rounding; a padding row (seq_len 1, fewer than its tokens) attends its own tokens only and stays finite."""
+    from sglang_neuron_amd import ops
+
+    B, S, H, G, d, P = 3, 4, 8, 2, 128, 16
+    lens = [1500, 400, 4]
+    q, kc, vc, table, kn, vn, slots = _multi_inputs(6, B, S, H, G, d, P, lens)
+    announce("gqa multi device lengths")
+    dev = lambda *ts: [t.cuda() for t in ts]  # noqa: E731
+    qd, kcd, vcd, td, knd, vnd, sd = dev(q, kc, vc, table, kn, vn, slots)
+    ld = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    kw = dict(sm_scale=d ** -0.5, new_slots=sd)
+    exact = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, host_seq_lens=lens, **kw)
+    bound = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, **kw)
+    torch.cuda.synchronize()
+    assert_close_attn(bound.cpu(), exact.cpu(), "bound plan")
+    ld[2] = 1
+    sd[2] = 0
+    pad = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(pad[:2], bound[:2]) and bool(torch.isfinite(pad).all())
