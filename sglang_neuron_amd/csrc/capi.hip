@@ -266,8 +266,13 @@ int sna_plan_decode(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32
   const int64_t target = kind == 0 ? (int64_t)cus * (depth >= 3 ? 2 : 8) : (int64_t)cus;
   const int64_t items_target = std::max<int64_t>(1, target / ctas_per_item);
   int32_t split_tiles = (int32_t)std::max<int64_t>(waves, (total_tiles + items_target - 1) / items_target);
-  // short rows (a sliding window, a few pages) stay whole: one split, no combine pass
+  // short rows (a sliding window, a few pages) stay whole: one split, no combine pass. Rows of up to 12 tiles always
+  // (graph replays, 16 / 8 heads of 128, bf16: one row of 10 tiles 8.5 -> 7.7 us, eight of 12 tiles 10.0 -> 9.8; of 14,
+  // 10.3 -> 11.4), of up to 24 where the whole rows already give every CU a workgroup (32 rows of up to 24 tiles, 32 / 8
+  // heads, FP8: 16.4 -> 12.1 us; of 16 tiles, bf16, 16.8 -> 14.3)
   split_tiles = std::max(split_tiles, std::min(max_tiles, 2 * waves));
+  if (max_tiles <= 12 || (max_tiles <= 24 && (int64_t)B * ctas_per_item >= cus))
+    split_tiles = std::max(split_tiles, max_tiles);
   // A MLA split's row ids live in the kernel's LDS, which caps it at kMlaMaxSplitTiles tiles.
   constexpr int32_t kMlaMaxSplitTiles = kMlaMaxSplitKeys / 16;
   const int32_t cap = kind != 0 ? kMlaMaxSplitTiles : std::max(max_tiles, waves);
