@@ -4,15 +4,20 @@
 //   reference: models/glm52/kernels/decode/attention/indexer/indexer_torch.py (pack_indexer_keys_fp8 :44-53, the
 //   score of indexer_kv_score_torch_ref :254-268, indexer_topk_local_torch_ref :296-309)
 //
-// Score: one workgroup of 4 waves per (row, 2048 keys); each wave takes 16-key tiles. S[head, key] = Q . K^T on
+// Score: one workgroup of 4 waves per (row, run of up to 4096 keys); each wave takes 16-key tiles. Bound by its key
+// loads (268 MB at about 5.2 TB/s on 16 rows of 131072 keys; with non-temporal loads, more waves or a deeper ring the
+// same). S[head, key] = Q . K^T on
 // v_mfma_scale_f32_16x16x128_f8f6f4 (one instruction covers d = 128): lane (g4, i) feeds row i of the head tile (the
 // query split exactly into two e4m3fn parts, hi + lo / 16, of a power-of-two-scaled row, whose E8M0 A scales undo
-// the scaling) and column i, the 32 key bytes 32 g4 .. + 31 of key i, loaded straight from HBM into a register ring.
+// the scaling) and column i, key i's bytes 16 g4 .. + 15 and 64 + 16 g4 .. + 15, loaded straight from HBM into a
+// register ring.
 // The result hands lane (g4, i) heads 4 g4 + r of key i: the head-weighted ReLU sum is 16 terms in the lane, then a
 // sum over the four lane groups. Bytes per key: 128 (the fp8 row) + 2 (the bf16 score written).
 //
 // Top-k: a two-byte radix select over order-preserving 16-bit keys of the scores, the row cut into segments of 8192
 // scores, in four launches that publish per-segment histograms and counts to a workspace (described below).
+
+#include <algorithm>
 
 #include "sna_device.h"
 #include "sna_host.h"
@@ -32,6 +37,7 @@ struct IndexerArgs {
   uint16_t* out;          // [B, width] bf16 (row stride out_stride)
   int64_t out_stride;
   int32_t B, H, width, P;
+  int32_t keys_wg;  // keys per workgroup
   int64_t num_blocks;
   float scale;  // d^-0.5
 };
@@ -44,21 +50,26 @@ __device__ __forceinline__ f32x4_t mfma_16x16x128_fp8_sa(const uint32_t (&a)[8],
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, scale_a, 0, 127);
 }
 
-constexpr int kScoreKeys = 2048;  // keys per workgroup (a multiple of 64): 32 tiles of 16 keys per wave
+// Keys per workgroup: a multiple of kScoreStep (PD steps of the four waves' 64 keys), at most kScoreKeys. The host picks
+// the number that gives the launch about kScoreBlocks workgroups, two a CU, in one round: 16 rows of 131072 keys (64
+// heads), store, scores and top-k 77.8 -> 74.5 us against 2048 keys a workgroup in two rounds (768 workgroups 79.7, 1024
+// 80.7, 1536 85.5 with the non-temporal loads), one row of 131072 or four of 32768 31.5 -> 26.5.
+constexpr int kScoreKeys = 4096, kScoreStep = 256, kScoreBlocks = 512;
 
 template <int HT>  // head tiles of 16
 __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
   // PD: key tiles each wave has in flight ahead of the one it scores (fewer with 128 heads, whose query operands
   // take 128 VGPRs)
-  constexpr int D = 128, TILES = kScoreKeys / 64, PD = HT >= 8 ? 2 : 4;
-  static_assert(kScoreKeys % 64 == 0 && kScoreKeys / 64 <= 32, "a 32-bit mask of live tiles");
+  constexpr int D = 128, PD = HT >= 8 ? 2 : 4;
+  static_assert(kScoreStep % (64 * PD) == 0 && kScoreKeys % kScoreStep == 0, "whole turns of the ring");
   __shared__ uint32_t sm_q[HT][2][8][64];  // [head tile][hi, lo][dword][lane]: the MFMA A operand of each lane
   __shared__ int32_t sm_ex[HT][64];         // floor(log2 amax) of the head lane (li) feeds, per head tile
+  __shared__ int32_t sm_row[kScoreKeys];    // the keys' byte offsets in the cache / 16 (under 2^31), -1: dead
   __shared__ __align__(16) uint16_t sm_out[kScoreKeys];  // the workgroup's bf16 scores
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int32_t b = blockIdx.y;
-  const int32_t e_blk = (int32_t)blockIdx.x * kScoreKeys;
+  const int32_t e_blk = (int32_t)blockIdx.x * a.keys_wg;
   if (e_blk >= a.width) return;
   const int32_t limit = a.limits[b];
   const int32_t* trow = a.table + (int64_t)b * a.table_stride;
@@ -70,50 +81,41 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
   for (int j = 0; j < QT; ++j) {
     const int ht = wave + 4 * j;
     if (ht < HT) {
-      const uint16_t* qp = a.q + ((int64_t)b * a.H + 16 * ht + li) * D + 32 * g4;
+      const uint16_t* qp = a.q + ((int64_t)b * a.H + 16 * ht + li) * D + 16 * g4;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) qraw[j][c] = ld16(qp + 8 * c);
+      for (int c = 0; c < 4; ++c) qraw[j][c] = ld16(qp + 64 * (c >> 1) + 8 * (c & 1));
     }
   }
 
-  // This lane's key of tile t is e_blk + 64 t + 16 wave + li (the four waves cover 64 consecutive keys per step);
-  // its page is looked up first, all tiles at once. Bit t of live_bits: the key is resident, its page valid.
-  // (col, off) = divmod(e, P), stepped by 64 keys per tile: one division for the first tile, then
-  // (col, off) += divmod(64, P) with at most one carry.
-  int32_t kofs[TILES];  // the key row's byte offset in the cache / 16 (the cache is under 2^35 bytes), if live
-  uint32_t live_bits = 0;
+  // The keys' rows: thread t resolves keys e_blk + t, + 256, ..., eight lookups in flight. (col, off) = divmod(e, P),
+  // stepped by 256 keys: one division for the first, then (col, off) += divmod(256, P) with at most one carry.
   {
-    const int32_t e0 = e_blk + 16 * wave + li, step_col = 64 / a.P, step_off = 64 % a.P;
+    const int32_t e0 = e_blk + tid, step_col = 256 / a.P, step_off = 256 % a.P;
     int32_t col = e0 / a.P, off = e0 - col * a.P;
+    for (int32_t i0 = 0; i0 < a.keys_wg; i0 += 8 * 256) {
+      int32_t page[8], poff[8];
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-      const int32_t e = e0 + 64 * t;
-      const int32_t page = (e < a.width && col < a.table_width) ? trow[col] : -1;
-      const bool live = e < limit && page >= 0 && (int64_t)page < a.num_blocks;
-      live_bits |= live ? (1u << t) : 0u;
-      kofs[t] = live ? (int32_t)((((int64_t)page * a.P + off) * D) >> 4) : 0;
-      col += step_col;
-      off += step_off;
-      if (off >= a.P) off -= a.P, ++col;
+      for (int u = 0; u < 8; ++u) {
+        const int32_t e = e0 + i0 + 256 * u;
+        page[u] = (i0 + 256 * u < a.keys_wg && e < a.width && e < limit && col < a.table_width) ? trow[col] : -1;
+        poff[u] = off;
+        col += step_col;
+        off += step_off;
+        if (off >= a.P) off -= a.P, ++col;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const bool live = page[u] >= 0 && (int64_t)page[u] < a.num_blocks;
+        if (i0 + 256 * u < a.keys_wg)
+          sm_row[i0 + 256 * u + tid] = live ? (int32_t)((((int64_t)page[u] * a.P + poff[u]) * D) >> 4) : -1;
+      }
     }
   }
 
-  // key tiles in flight: tile t's 32 bytes of this lane land in ring[t % PD]. Every lane loads (a dead key reads
-  // row 0 of the cache, in bounds, and its score is replaced), so no branch or store sits between a load and its
-  // use and the waits count only the ring's own loads.
-  uint32_t ring[PD][8];
-  auto fetch = [&](int t, uint32_t (&kb)[8]) {
-    const uint8_t* kp = a.keys + ((int64_t)kofs[t] << 4) + 32 * g4;
-    // plain loads: with the non-temporal hint the same stream measured ~3% slower
-    const uint4 x0 = ld16(kp), x1 = ld16(kp + 16);
-    kb[0] = x0.x, kb[1] = x0.y, kb[2] = x0.z, kb[3] = x0.w, kb[4] = x1.x, kb[5] = x1.y, kb[6] = x1.z, kb[7] = x1.w;
-  };
-#pragma unroll
-  for (int u = 0; u < PD; ++u) fetch(u, ring[u]);
-
-  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 32 g4 .. + 31, as two exact
-  // e4m3fn parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over the head's 128 dims); the E8M0 A
-  // scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w, w + 4, ... into LDS.
+  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 16 g4 .. + 15 and 64 + 16 g4 .. + 15
+  // (the key bytes it loads), as two exact e4m3fn parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over
+  // the head's 128 dims); the E8M0 A scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w,
+  // w + 4, ... into LDS.
 #pragma unroll
   for (int j = 0; j < QT; ++j) {
     const int ht = wave + 4 * j;
@@ -154,6 +156,23 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     for (int r = 0; r < 4; ++r) wl[ht][r] = a.w[(int64_t)b * a.H + 16 * ht + 4 * g4 + r] * a.scale;
 
   __syncthreads();
+  // Key tiles in flight: tile t's (keys 64 t + 16 wave + li) 32 bytes of this lane land in ring[t % PD], its row offset in
+  // kof[t % PD]; an instruction reads 64 contiguous bytes of each of 16 keys. Every lane loads (a dead key reads row 0 of
+  // the cache, in bounds, and its score is replaced), so no branch or store sits between a load and its use and the
+  // waits count only the ring's own loads. Plain loads: with the non-temporal hint 16 rows of 65536 keys, half of them in
+  // the Infinity Cache, took 49.5 us instead of 45.7 (16 of 131072 the same).
+  const int32_t tiles = a.keys_wg / 64;
+  uint32_t ring[PD][8];
+  int32_t kof[PD];
+  auto fetch = [&](int32_t t, int u) {
+    kof[u] = sm_row[64 * t + 16 * wave + li];
+    const uint8_t* kp = a.keys + ((int64_t)max(kof[u], 0) << 4) + 16 * g4;
+    const uint4 x0 = ld16(kp), x1 = ld16(kp + 64);
+    ring[u][0] = x0.x, ring[u][1] = x0.y, ring[u][2] = x0.z, ring[u][3] = x0.w;
+    ring[u][4] = x1.x, ring[u][5] = x1.y, ring[u][6] = x1.z, ring[u][7] = x1.w;
+  };
+#pragma unroll
+  for (int u = 0; u < PD; ++u) fetch(u, u);
   uint32_t qhi[HT][8], qlo[HT][8];
   int32_t sc_hi[HT], sc_lo[HT];
 #pragma unroll
@@ -166,28 +185,31 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
   }
 
   // scores of the workgroup's keys, written out coalesced at the end
+  for (int32_t t0 = 0; t0 < tiles; t0 += PD) {
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) {
-    float sum = 0.0f;
+    for (int u = 0; u < PD; ++u) {
+      float sum = 0.0f;
 #pragma unroll
-    for (int ht = 0; ht < HT; ++ht) {
-      f32x4_t s = {0.f, 0.f, 0.f, 0.f};
-      s = mfma_16x16x128_fp8_sa(qhi[ht], ring[t % PD], s, sc_hi[ht]);
-      s = mfma_16x16x128_fp8_sa(qlo[ht], ring[t % PD], s, sc_lo[ht]);
+      for (int ht = 0; ht < HT; ++ht) {
+        f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+        s = mfma_16x16x128_fp8_sa(qhi[ht], ring[u], s, sc_hi[ht]);
+        s = mfma_16x16x128_fp8_sa(qlo[ht], ring[u], s, sc_lo[ht]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)  // relu as an integer max: a negative float's bits are a negative integer
-        sum = fmaf(wl[ht][r], __int_as_float(max(__float_as_int(s[r]), 0)), sum);
+        for (int r = 0; r < 4; ++r)  // relu as an integer max: a negative float's bits are a negative integer
+          sum = fmaf(wl[ht][r], __int_as_float(max(__float_as_int(s[r]), 0)), sum);
+      }
+      const bool live = kof[u] >= 0;
+      fetch(min(t0 + u + PD, tiles - 1), u);  // (past the last tile: it again, not used)
+      sum = sum_across_groups(sum);  // every lane of key li holds the key's sum
+      sm_out[64 * (t0 + u) + 16 * wave + li] =
+          (uint16_t)f32_to_bf16_bits(live ? fminf(sum, kIndexMaskBound) : -kIndexMaskBound);
     }
-    if (t + PD < TILES) fetch(t + PD, ring[t % PD]);
-    sum = sum_across_groups(sum);  // every lane of key li holds the key's sum
-    const bool live = (live_bits >> t) & 1u;
-    sm_out[64 * t + 16 * wave + li] = (uint16_t)f32_to_bf16_bits(live ? fminf(sum, kIndexMaskBound) : -kIndexMaskBound);
   }
   __syncthreads();
   uint16_t* orow = a.out + (int64_t)b * a.out_stride + e_blk;
-  const int32_t n = min(kScoreKeys, a.width - e_blk);
-  if (n == kScoreKeys && ((uintptr_t)orow & 7) == 0) {
-    for (int32_t i = 4 * tid; i < kScoreKeys; i += 4 * 256)
+  const int32_t n = min(a.keys_wg, a.width - e_blk);
+  if (n == a.keys_wg && ((uintptr_t)orow & 7) == 0) {
+    for (int32_t i = 4 * tid; i < n; i += 4 * 256)
       *reinterpret_cast<uint2*>(orow + i) = *reinterpret_cast<const uint2*>(&sm_out[i]);
   } else {
     for (int32_t i = tid; i < n; i += 256) orow[i] = sm_out[i];
@@ -494,7 +516,10 @@ int sna_indexer_scores(const void* q, const float* w, const uint8_t* keys, const
   a.P = page_size;
   a.num_blocks = num_blocks;
   a.scale = 1.0f / sqrtf((float)head_dim);
-  const dim3 grid((unsigned)((width + kScoreKeys - 1) / kScoreKeys), (unsigned)B);
+  const int64_t per = ((int64_t)B * width + kScoreBlocks - 1) / kScoreBlocks;
+  a.keys_wg = (int32_t)std::min<int64_t>(kScoreKeys, std::max<int64_t>(2 * kScoreStep,
+                                                                      (per + kScoreStep - 1) / kScoreStep * kScoreStep));
+  const dim3 grid((unsigned)((width + a.keys_wg - 1) / a.keys_wg), (unsigned)B);
   const hipStream_t s = (hipStream_t)stream;
   switch (num_heads / 16) {
     case 1: hipLaunchKernelGGL((indexer_score_kernel<1>), grid, dim3(256), 0, s, a); break;
