@@ -9,8 +9,7 @@
 // same). S[head, key] = Q . K^T on
 // v_mfma_scale_f32_16x16x128_f8f6f4 (one instruction covers d = 128): lane (g4, i) feeds row i of the head tile (the
 // query split exactly into two e4m3fn parts, hi + lo / 16, of a power-of-two-scaled row, whose E8M0 A scales undo
-// the scaling) and column i, key i's bytes 16 g4 .. + 15 and 64 + 16 g4 .. + 15, loaded straight from HBM into a
-// register ring.
+// the scaling) and column i, the 32 key bytes 32 g4 .. + 31 of key i, loaded straight from HBM into a register ring.
 // The result hands lane (g4, i) heads 4 g4 + r of key i: the head-weighted ReLU sum is 16 terms in the lane, then a
 // sum over the four lane groups. Bytes per key: 128 (the fp8 row) + 2 (the bf16 score written).
 //
@@ -81,9 +80,9 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
   for (int j = 0; j < QT; ++j) {
     const int ht = wave + 4 * j;
     if (ht < HT) {
-      const uint16_t* qp = a.q + ((int64_t)b * a.H + 16 * ht + li) * D + 16 * g4;
+      const uint16_t* qp = a.q + ((int64_t)b * a.H + 16 * ht + li) * D + 32 * g4;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) qraw[j][c] = ld16(qp + 64 * (c >> 1) + 8 * (c & 1));
+      for (int c = 0; c < 4; ++c) qraw[j][c] = ld16(qp + 8 * c);
     }
   }
 
@@ -112,8 +111,7 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     }
   }
 
-  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 16 g4 .. + 15 and 64 + 16 g4 .. + 15
-  // (the key bytes it loads), as two exact e4m3fn parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over
+  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 32 g4 .. + 31, as two exact e4m3fn parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over
   // the head's 128 dims); the E8M0 A scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w,
   // w + 4, ... into LDS.
 #pragma unroll
@@ -157,17 +155,17 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
 
   __syncthreads();
   // Key tiles in flight: tile t's (keys 64 t + 16 wave + li) 32 bytes of this lane land in ring[t % PD], its row offset in
-  // kof[t % PD]; an instruction reads 64 contiguous bytes of each of 16 keys. Every lane loads (a dead key reads row 0 of
-  // the cache, in bounds, and its score is replaced), so no branch or store sits between a load and its use and the
-  // waits count only the ring's own loads. Plain loads: with the non-temporal hint 16 rows of 65536 keys, half of them in
+  // kof[t % PD]. Every lane loads (a dead key reads row 0 of the cache, in bounds, and its score is replaced), so no
+  // branch or store sits between a load and its use and the waits count only the ring's own loads. (Instructions of 64
+  // contiguous bytes a key measured the same, and sum the dims in another order.) Plain loads: with the non-temporal hint 16 rows of 65536 keys, half of them in
   // the Infinity Cache, took 49.5 us instead of 45.7 (16 of 131072 the same).
   const int32_t tiles = a.keys_wg / 64;
   uint32_t ring[PD][8];
   int32_t kof[PD];
   auto fetch = [&](int32_t t, int u) {
     kof[u] = sm_row[64 * t + 16 * wave + li];
-    const uint8_t* kp = a.keys + ((int64_t)max(kof[u], 0) << 4) + 16 * g4;
-    const uint4 x0 = ld16(kp), x1 = ld16(kp + 64);
+    const uint8_t* kp = a.keys + ((int64_t)max(kof[u], 0) << 4) + 32 * g4;
+    const uint4 x0 = ld16(kp), x1 = ld16(kp + 16);
     ring[u][0] = x0.x, ring[u][1] = x0.y, ring[u][2] = x0.z, ring[u][3] = x0.w;
     ring[u][4] = x1.x, ring[u][5] = x1.y, ring[u][6] = x1.z, ring[u][7] = x1.w;
   };
