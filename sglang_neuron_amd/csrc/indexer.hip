@@ -14,7 +14,7 @@
 // sum over the four lane groups. Bytes per key: 128 (the fp8 row) + 2 (the bf16 score written).
 //
 // Top-k: a two-byte radix select over order-preserving 16-bit keys of the scores, the row cut into segments of 8192
-// scores, in four launches that publish per-segment histograms and counts to a workspace (described below).
+// scores, in three launches that publish per-segment histograms to a workspace (described below).
 
 #include <algorithm>
 
@@ -220,31 +220,29 @@ __device__ __forceinline__ uint32_t key_bits(uint32_t key) { return (key & 0x800
 
 // ---- top-k: a two-byte radix select over the rows' segments ----
 // A row of bf16 scores is cut into segments of kTopkSeg scores, one workgroup of 1024 lanes (8 scores each, one
-// 16-byte load) per (segment, row). Scores compare through order_key, a 16-bit key that sorts as the value does. Four
+// 16-byte load) per (segment, row). Scores compare through order_key, a 16-bit key that sorts as the value does. Three
 // launches, each workgroup reading only what earlier launches published in the workspace (no zeroing, no global
-// atomics):
+// atomics); they are bound by launch and round trips (about 5 us each on 16 rows of 131072), so a segment's counts above
+// and at the threshold come from its two histograms, where a fourth launch used to count them:
 //   topk_hist_hi:  the segment's histogram of the key's high byte          -> hist_hi[b][s][256]
 //   topk_hist_lo:  the row's bin H holding the k-th largest key (summing hist_hi over the segments);
 //                  the segment's histogram of the low byte of keys in H    -> hist_lo[b][s][256]
-//   topk_count:    the threshold key T (the k-th largest) and the count above it; the segment's counts of keys
-//                  above and equal to T                                    -> counts[b][s], and sel[b] from s = 0
-//   topk_write:    positions in order: keys above T at the running count of those before them, then T's ties at
-//                  n_above + their running count, while that is below k.
-// Workspace per row: (2 * 256 + 1) * S + 4 u32, S = ceil(width / kTopkSeg).
+//   topk_write:    the threshold key T (the k-th largest) and the count above it; positions in order: keys above T at
+//                  the running count of those before them (earlier segments' from their histograms), then T's ties
+//                  at n_above + their running count, while that is below k.
+// Workspace per row: (2 * 256 + 1) * S + 4 u32, S = ceil(width / kTopkSeg) (the last S + 4 unused).
 constexpr int kTopkSeg = 8192, kTopkCopies = 32;
 
 struct TopkRow {
   const uint16_t* row;  // this row's scores
   uint32_t* hist_hi;    // [S][256]
   uint32_t* hist_lo;    // [S][256]
-  uint32_t* counts;     // [S]: (ties << 16) | above
-  uint32_t* sel;        // [4]: T, n_above
 };
 
 __device__ __forceinline__ TopkRow topk_row(const uint16_t* scores, int64_t score_stride, uint32_t* ws, int32_t S) {
   const int32_t b = blockIdx.y;
   uint32_t* base = ws + (int64_t)b * ((2 * 256 + 1) * (int64_t)S + 4);
-  return {scores + (int64_t)b * score_stride, base, base + 256 * S, base + 512 * S, base + 513 * S};
+  return {scores + (int64_t)b * score_stride, base, base + 256 * S};
 }
 
 // this lane's 8 keys of segment blockIdx.x (past the row: key 0, never counted); in[j] says whether key j is inside
@@ -282,11 +280,14 @@ __device__ __forceinline__ void topk_publish(const uint32_t* hist, uint32_t* dst
 
 // The bin (from the top) where the running count of the row's keys, over the S published histograms hist[S][256],
 // reaches `need`, and the count in the bins above it plus base_above; every lane gets both. Threads 0..255 take
-// bin 255 - t. wtot: 4 u32 of LDS, out: 2 u32 of LDS.
+// bin 255 - t; `prior` is the thread's bin's count in the segments before this workgroup's. wtot: 4 u32 of LDS, out: 2
+// u32 of LDS.
 __device__ __forceinline__ void topk_pick(const uint32_t* hist, int32_t S, uint32_t need, uint32_t base_above,
-                                          uint32_t* wtot, uint32_t* out, uint32_t& bin, uint32_t& above) {
+                                          uint32_t* wtot, uint32_t* out, uint32_t& bin, uint32_t& above,
+                                          uint32_t& prior) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   uint32_t cnt = 0, incl = 0;
+  prior = 0;
   if (t < 256) {
     // S published histograms, written by other workgroups (other XCDs): 16 independent loads in flight at a time
     for (int32_t s0 = 0; s0 < S; s0 += 16) {
@@ -294,7 +295,7 @@ __device__ __forceinline__ void topk_pick(const uint32_t* hist, int32_t S, uint3
 #pragma unroll
       for (int j = 0; j < 16; ++j) v[j] = s0 + j < S ? hist[(int64_t)(s0 + j) * 256 + 255 - t] : 0u;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) cnt += v[j];
+      for (int j = 0; j < 16; ++j) cnt += v[j], prior += s0 + j < (int32_t)blockIdx.x ? v[j] : 0u;
     }
     incl = cnt;
 #pragma unroll
@@ -347,8 +348,8 @@ __global__ __launch_bounds__(1024) void topk_hist_lo_kernel(const uint16_t* __re
   uint32_t key[8];
   topk_keys(r.row, topk_vec(scores, score_stride), width, key);
   topk_clear(hist);
-  uint32_t hi, above;
-  topk_pick(r.hist_hi, S, (uint32_t)k, 0, wtot, pick, hi, above);  // its barriers also cover the clear
+  uint32_t hi, above, prior;
+  topk_pick(r.hist_hi, S, (uint32_t)k, 0, wtot, pick, hi, above, prior);  // its barriers also cover the clear
   uint32_t* mine = hist + (threadIdx.x & (kTopkCopies - 1));
   const int32_t e = blockIdx.x * kTopkSeg + 8 * threadIdx.x;
 #pragma unroll
@@ -358,68 +359,32 @@ __global__ __launch_bounds__(1024) void topk_hist_lo_kernel(const uint16_t* __re
   topk_publish(hist, r.hist_lo + (int64_t)blockIdx.x * 256);
 }
 
-// the threshold key T and the count above it, from the two published histograms
-__device__ __forceinline__ void topk_threshold(const TopkRow& r, int32_t S, int32_t k, uint32_t* wtot, uint32_t* pick,
-                                               uint32_t& T, uint32_t& n_above) {
-  uint32_t hi, above1, lo;
-  topk_pick(r.hist_hi, S, (uint32_t)k, 0, wtot, pick, hi, above1);
-  __syncthreads();  // pick[] is rewritten
-  topk_pick(r.hist_lo, S, (uint32_t)k, above1, wtot, pick, lo, n_above);
-  T = (hi << 8) | lo;
-}
-
-__global__ __launch_bounds__(1024) void topk_count_kernel(const uint16_t* __restrict__ scores, int64_t score_stride,
-                                                          int32_t width, int32_t S, int32_t k,
-                                                          uint32_t* __restrict__ ws) {
-  __shared__ uint32_t wtot[16], pick[2];
-  const TopkRow r = topk_row(scores, score_stride, ws, S);
-  uint32_t key[8];
-  topk_keys(r.row, topk_vec(scores, score_stride), width, key);
-  uint32_t T, n_above;
-  topk_threshold(r, S, k, wtot, pick, T, n_above);
-  const int32_t e = blockIdx.x * kTopkSeg + 8 * threadIdx.x;
-  uint32_t cnt = 0;  // (ties << 16) | above, each at most 8 per lane and kTopkSeg per segment
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const bool in = e + j < width;
-    cnt += (in && key[j] > T) ? 1u : 0u;
-    cnt += (in && key[j] == T) ? 0x10000u : 0u;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-  __syncthreads();  // wtot was read by the picks
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) wtot[wave] = cnt;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t total = 0;
-    for (int w = 0; w < 16; ++w) total += wtot[w];
-    r.counts[blockIdx.x] = total;
-    if (blockIdx.x == 0) {
-      r.sel[0] = T;
-      r.sel[1] = n_above;
-    }
-  }
-}
-
 __global__ __launch_bounds__(1024) void topk_write_kernel(const uint16_t* __restrict__ scores, int64_t score_stride,
                                                           int32_t width, int32_t S, int32_t k,
                                                           uint32_t* __restrict__ ws, int32_t* __restrict__ out,
                                                           int64_t out_stride) {
-  __shared__ uint32_t wtot[16];
+  __shared__ uint32_t wtot[16], pick[2], before_gt[4], before_eq;
   const TopkRow r = topk_row(scores, score_stride, ws, S);
   uint32_t key[8];
   topk_keys(r.row, topk_vec(scores, score_stride), width, key);
-  const uint32_t T = r.sel[0], n_above = r.sel[1], n_ties = (uint32_t)k - n_above;
-  uint32_t run_gt = 0, run_eq = 0;  // the counts of the segments before this one (ties may pass 16 bits here)
-  for (int32_t s0 = 0; s0 < (int32_t)blockIdx.x; s0 += 16) {
-    uint32_t c[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) c[j] = s0 + j < (int32_t)blockIdx.x ? r.counts[s0 + j] : 0u;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) run_gt += c[j] & 0xffffu, run_eq += c[j] >> 16;
-  }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the threshold key T and the count above it, from the two published histograms
+  uint32_t hi, above1, lo, n_above, prior_hi, prior_lo;
+  topk_pick(r.hist_hi, S, (uint32_t)k, 0, wtot, pick, hi, above1, prior_hi);
+  __syncthreads();  // pick[] is rewritten
+  topk_pick(r.hist_lo, S, (uint32_t)k, above1, wtot, pick, lo, n_above, prior_lo);
+  const uint32_t T = (hi << 8) | lo, n_ties = (uint32_t)k - n_above;
+  // the counts above and equal to T in the segments before this one: their bins above hi, and above and at lo
+  if (tid < 256) {
+    const uint32_t bin = 255u - (uint32_t)tid;
+    uint32_t gt = (bin > hi ? prior_hi : 0u) + (bin > lo ? prior_lo : 0u);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) gt += __shfl_xor(gt, off, 64);
+    if (lane == 0) before_gt[wave] = gt;
+    if (bin == lo) before_eq = prior_lo;
+  }
+  __syncthreads();
+  const uint32_t run_gt = before_gt[0] + before_gt[1] + before_gt[2] + before_gt[3], run_eq = before_eq;
   const int32_t e = blockIdx.x * kTopkSeg + 8 * tid;
   uint32_t cnt = 0;
 #pragma unroll
@@ -557,7 +522,6 @@ int sna_topk_positions(const void* scores, int64_t score_stride, int32_t B, int3
   hipLaunchKernelGGL(topk_hist_hi_kernel, grid, block, 0, st, sc, score_stride, width, S, ws);
   hipLaunchKernelGGL(topk_hist_lo_kernel, grid, block, 0, st, sc, score_stride, width, S, k,
                         ws);
-  hipLaunchKernelGGL(topk_count_kernel, grid, block, 0, st, sc, score_stride, width, S, k, ws);
   hipLaunchKernelGGL(topk_write_kernel, grid, block, 0, st, sc, score_stride, width, S, k, ws, out,
                         out_stride);
   return check_launch("topk_positions");
