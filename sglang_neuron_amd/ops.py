@@ -568,8 +568,8 @@ def paged_decode_gqa_multi(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     k_new = _contig(k_new, "k_new", torch.bfloat16)
     v_new = _contig(v_new, "v_new", torch.bfloat16)
     slots = _contig(_as(new_slots.reshape(-1), torch.int64), "new_slots")
-    _need(block_table.dim() == 2 and block_table.shape[0] == B, lambda: f"block_table must be [{B}, width]")
-    table = _as(block_table, torch.int32)
+    _need(block_table.dim() == 2 and block_table.shape[0] >= B, lambda: f"block_table must be [{B}, width]")
+    table = _as(block_table[:B], torch.int32)  # (a table of more rows: a padded batch's)
     table = table if table.stride(1) == 1 else table.contiguous()
     lens = _contig(_as(seq_lens.reshape(-1), torch.int32), "seq_lens")
     _need(lens.numel() == B, lambda: f"{lens.numel()} seq_lens for {B} rows")

@@ -291,6 +291,12 @@ def test_gqa_multi_device_lengths_and_padding_rows():
     bound = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, **kw)
     torch.cuda.synchronize()
     assert_close_attn(bound.cpu(), exact.cpu(), "bound plan")
+    # a table of a padded batch: rows past B are not read, whatever the columns' stride
+    wide = torch.full((B + 2, td.shape[1]), 1 << 20, dtype=torch.int64, device="cuda")
+    wide[:B] = td
+    for table_ in (wide, wide.t().contiguous().t()):
+        more = ops.paged_decode_gqa_multi(qd, kcd, vcd, table_, ld, knd, vnd, host_seq_lens=lens, **kw)
+        assert torch.equal(more, exact)
     ld[2] = 1
     sd[2] = 0
     pad = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, **kw)
