@@ -248,8 +248,8 @@ __device__ __forceinline__ void wave_incl_scan4(uint32_t (&v)[4]) {
 // arithmetic is deterministic, so every workgroup gets the same one): the rows' key counts (seq_len - 1, held to the
 // table's width and the stream's 65535 tiles per row) into keys[b]; the ranges' starts into cs[w] (cs[w] = the
 // stream's end for w at or past the split's n, and cs[256] too); row << 16 | tile offset into cro[w]; n into *n_out.
-// With a workgroup for every row (B <= n, n = min(launched workgroups, tiles)) rows are apportioned whole: the least
-// piece length T with sum_b ceil(tiles_b / T) <= n is found by bisection, and row b is cut into ceil(tiles_b / T)
+// With a workgroup for every row (B <= n, n = min(launched workgroups, the rows' stream_pieces)) rows are apportioned
+// whole: the least piece length T with sum_b ceil(tiles_b / T) <= n is found by bisection, and row b is cut into ceil(tiles_b / T)
 // equal pieces (the same longest piece as the host planner's greedy apportionment, within a tile); otherwise the
 // stream is cut into n equal ranges. tmp: 5 x 256 words of LDS scratch.
 __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int32_t* keys, int32_t* n_out,
@@ -257,7 +257,7 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
   const int lane = threadIdx.x & 63;
   const int32_t B = a.B;
   const int32_t kmax = (int32_t)min((int64_t)a.table_width * a.P, (int64_t)65535 * 16);
-  uint32_t tiles[4], first[4], mx = 0;
+  uint32_t tiles[4], first[4], mx = 0, worth = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int32_t r = lane + 64 * i;
@@ -269,6 +269,7 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
     }
     first[i] = tiles[i];
     mx = max(mx, tiles[i]);
+    worth += (uint32_t)stream_pieces((int32_t)tiles[i]);
   }
   wave_incl_scan4(first);
   uint32_t total = 0;
@@ -278,7 +279,8 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
     first[i] = total + first[i] - tiles[i];
     total += part;
   }
-  const uint32_t n = min((uint32_t)gridDim.x, total);
+  mx = (uint32_t)wave_max((float)mx);
+  const uint32_t n = min((uint32_t)gridDim.x, mx <= kStreamWholeTiles ? (uint32_t)B : (uint32_t)wave_sum((float)worth));
   uint32_t* t_first = tmp;
   uint32_t* t_tiles = tmp + 256;
   uint32_t* t_pieces = tmp + 512;
@@ -297,7 +299,6 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
   const bool whole = (uint32_t)B <= n;
   uint32_t n_split = n;
   if (whole) {
-    mx = (uint32_t)wave_max((float)mx);
     uint32_t lo = max(1u, (total + n - 1) / n), hi = mx;
     if (n > (uint32_t)B) hi = min(hi, (total + (n - B) - 1) / (n - B));  // feasible: sum <= total / T + B <= n
     lo = min(lo, hi);

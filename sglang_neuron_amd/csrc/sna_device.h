@@ -25,6 +25,20 @@ constexpr int kGqaDevSplitRows = 512;
 constexpr int kGqaDevSplitMaxTiles = (1 << 17) - 1;
 // The most keys one sparse (DSA) workgroup may resolve (their row ids live in the kernel's LDS); the planner keeps to it.
 constexpr int kMlaMaxSplitKeys = 2048;
+
+// The workgroups that a paged MLA row of so many 16-key tiles is worth; a launch runs at most the sum of its rows', the
+// longest pieces as short as that many allow. A workgroup's tile loop takes time in proportion to tiles / workgroups, the
+// row's merge (a 32 KB partial a workgroup, written and read again) in proportion to the workgroups, so their sum is least
+// at sqrt(k tiles); k = 3 from sweeps of the workgroup count (graph replays, FP8 / bf16 rows, 16 heads, us: one row of
+// 4000 keys, 250 tiles: 250 workgroups 41.4 / 42.3, 63 20.5 / 19.8, 32 18.3 / 17.2, 25 18.7 / 18.2, 11 20.7 / 21.9; one of
+// 16000: 256 42.7 / 44.6, 63 24.8 / 25.8, 32 25.7 / 28.7; four of 1300-2000: 256 24.7 / 24.2, 70 18.0 / 17.4, 18 22.7 /
+// 24.0; eight of 670-1000: 256 20.4 / 18.9, 105 17.1 / 15.9, 35 19.3 / 19.3). A batch of rows of up
+// to 12 tiles, three a wave, stays whole and needs no merge (9 tiles, 32 rows: whole 14.6 / 13.6, six a row 17.5 / 15.3; 7 tiles, one row: 12.8 / 10.7, six
+// 15.9 / 13.1; at 13 tiles, one row: whole 15.2 / 14.2, eight 14.9 / 12.2).
+constexpr int32_t kStreamWholeTiles = 12;
+__host__ __device__ inline int32_t stream_pieces(int32_t tiles) {
+  return min(tiles, (int32_t)ceilf(sqrtf(3.0f * (float)tiles)));
+}
 // The MLA / DSA stream split's counter block at the start of its workspace: per (row, head group) an arrival counter
 // and a mask of merged latent blocks, then one count of finished workgroups, each in a 64-byte line of its own; zero
 // at rest. The last line holds a sticky status word: a launch that finds a counter past what a clean block allows

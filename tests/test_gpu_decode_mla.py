@@ -77,6 +77,29 @@ def test_mla_device_split_matches_oracle(name, over, bf16):
         assert torch.equal(scale.cpu(), scale_o), "row scales differ"
 
 
+# few rows: a row takes about sqrt(3 tiles) workgroups, one up to 12 tiles, cut on the host or on the device. (Tiles a
+# row: 1; 1, 2 and 3; 12, the longest whole row; 13; 4 and 13; a mixture; a long row.)
+@pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
+@pytest.mark.parametrize("lens", [[2], [17, 33, 34], [193], [194], [65, 209], [5000, 1, 60], [20001]], ids=str)
+def test_mla_few_rows_match_oracle(lens, bf16):
+    dev = torch.device("cuda", 0)
+    case = workloads.mla_case(overrides={"B": len(lens), "fixed_lens": lens})
+    want, cache_o, _ = mla_oracle(case, bf16=bf16)
+    table = case.block_table.to(dev)
+    exact = ops.plan_decode(1, case.B, host_seq_lens=case.seq_lens, ctas_per_item=1, num_cus=256)
+    bound = ops.plan_decode(1, case.B, max_seq_len=table.shape[1] * case.P, ctas_per_item=1, num_cus=256)
+    announce(f"mla few rows {lens} bf16={bf16}: n_ctas={exact.n_ctas}")
+    for plan in (exact, bound):
+        cache, scale = mla_gpu_pool(case, bf16=bf16)
+        out = ops.mla_decode(case.ql_nope.to(dev), case.q_pe.to(dev), cache, scale, table, case.seq_lens.to(dev),
+                             case.compact_new.to(dev), sm_scale=case.sm_scale, page_size=case.P,
+                             new_slots=case.new_slots.to(dev), plan=plan,
+                             host_seq_lens=None if plan.device_split else case.seq_lens)
+        torch.cuda.synchronize()
+        assert_close_attn(out, want, f"{lens} device_split={plan.device_split}")
+        assert torch.equal(cache.cpu().view(torch.uint8), cache_o.view(torch.uint8)), "row pool differs"
+
+
 # bf16 rows, the reference's DeepSeek-V2 pool (models/catalog.py:230-231: bf16 KV at page 128)
 MLA_BF16_CASES = [
     ("bf16-cfg3-page128", {"B": 8, "P": 128, "lens": (1024, 16384)}),
