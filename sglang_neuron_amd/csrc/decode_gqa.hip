@@ -616,7 +616,7 @@ void gqa_decode_kernel(GqaArgs a) {
 // e_s = exp2(m_s - M) and M the maximum over the splits and the sink. Lane s holds split s's weight; lane i holds the
 // head dims D / 64 * i .. + D / 64. The partials stream in chunks of 16 splits, each chunk's loads all in flight
 // together (the first before the weights are known).
-template <int D>
+template <int D, bool MULTI>
 __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
   constexpr int V = D / 64;
   constexpr int CH = 16;
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
     for (int v = 0; v < V; ++v) x[k][v] = k < S ? ob[k * sstride + v] : 0.0f;
   float2 ml = make_float2(-INFINITY, 0.0f);
   if (lane < S) ml = *reinterpret_cast<const float2*>(a.ws_ml + (row0 + (int64_t)lane * a.H) * 2);
-  const int32_t br = a.S == 1 ? b : b / a.S;  // the row of seq_lens (S tokens a row)
+  const int32_t br = MULTI ? b / a.S : b;  // the row of seq_lens (S tokens a row)
   const int32_t n = min(launched_splits(a, br, ld_const(a.seq_lens + br), a.dev_split ? *a.ws_st : a.split_tiles), S);
   if (n == 0) return;  // a row with no prior key: the lone-token kernel writes it
   const float m = lane < n ? ml.x : -INFINITY, l = lane < n ? ml.y : 0.0f;
@@ -669,11 +669,11 @@ __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
 }
 
 // Rows with no split at all (seq_len 1) get their output from this pass: only the own token (and the sink).
-template <int D, bool FP8>
+template <int D, bool FP8, bool MULTI>
 __global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgs a) {
   const int b = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
   // any split size counts the row's splits as nonzero iff it has a prior key
-  const int32_t br = a.S == 1 ? b : b / a.S;  // (S tokens a row)
+  const int32_t br = MULTI ? b / a.S : b;  // (S tokens a row)
   if (launched_splits(a, br, a.seq_lens[br], a.split_tiles) > 0) return;
   __shared__ float sm_kn[D], sm_vn[D];
   const float kstored = FP8 ? a.k_scale[g] : 1.0f, vstored = FP8 ? a.v_scale[g] : 1.0f;
@@ -746,8 +746,8 @@ static void launch_gqa(const GqaArgs& a, bool any_lone, hipStream_t s) {
       else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, false, 2, MULTI>), grid, dim3(256), 0, s, a);
     }
   }
-  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D>), dim3(a.B * a.S, a.H), dim3(64), 0, s, a);
-  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8>), dim3(a.B * a.S, a.G), dim3(128), 0, s, a);
+  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D, MULTI>), dim3(a.B * a.S, a.H), dim3(64), 0, s, a);
+  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8, MULTI>), dim3(a.B * a.S, a.G), dim3(128), 0, s, a);
 }
 
 template <int D, bool FP8>
