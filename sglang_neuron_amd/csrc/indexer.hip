@@ -13,8 +13,9 @@
 // The result hands lane (g4, i) heads 4 g4 + r of key i: the head-weighted ReLU sum is 16 terms in the lane, then a
 // sum over the four lane groups. Bytes per key: 128 (the fp8 row) + 2 (the bf16 score written).
 //
-// Top-k: a two-byte radix select over order-preserving 16-bit keys of the scores, the row cut into segments of 8192
-// scores, in three launches that publish per-segment histograms to a workspace (described below).
+// Top-k: a two-byte radix select over order-preserving 16-bit keys of the scores: rows of up to 16384 scores in one
+// workgroup each, longer ones cut into segments of 8192, in three launches that publish per-segment histograms to a
+// workspace (described below).
 
 #include <algorithm>
 
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     }
   }
 
-  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 32 g4 .. + 31, as two exact e4m3fn parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over
-  // the head's 128 dims); the E8M0 A scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w,
+  // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 32 g4 .. + 31, as two exact e4m3fn
+  // parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over the head's 128 dims); the E8M0 A scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w,
   // w + 4, ... into LDS.
 #pragma unroll
   for (int j = 0; j < QT; ++j) {
@@ -231,7 +232,7 @@ __device__ __forceinline__ uint32_t key_bits(uint32_t key) { return (key & 0x800
 //                  the running count of those before them (earlier segments' from their histograms), then T's ties
 //                  at n_above + their running count, while that is below k.
 // Workspace per row: (2 * 256 + 1) * S + 4 u32, S = ceil(width / kTopkSeg) (the last S + 4 unused).
-constexpr int kTopkSeg = 8192, kTopkCopies = 32;
+constexpr int kTopkSeg = 8192, kTopkCopies = 32, kTopkRowVecs = 2;
 
 struct TopkRow {
   const uint16_t* row;  // this row's scores
@@ -245,9 +246,8 @@ __device__ __forceinline__ TopkRow topk_row(const uint16_t* scores, int64_t scor
   return {scores + (int64_t)b * score_stride, base, base + 256 * S};
 }
 
-// this lane's 8 keys of segment blockIdx.x (past the row: key 0, never counted); in[j] says whether key j is inside
-__device__ __forceinline__ void topk_keys(const uint16_t* row, bool vec, int32_t width, uint32_t (&key)[8]) {
-  const int32_t e = blockIdx.x * kTopkSeg + 8 * threadIdx.x;
+// the 8 keys from position e (past the row: key 0, never counted)
+__device__ __forceinline__ void topk_keys(const uint16_t* row, bool vec, int32_t width, int32_t e, uint32_t (&key)[8]) {
   if (vec && e + 8 <= width) {
     const uint4 v = *reinterpret_cast<const uint4*>(row + e);
     const uint32_t x[4] = {v.x, v.y, v.z, v.w};
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(1024) void topk_hist_hi_kernel(const uint16_t* __re
   __shared__ uint32_t hist[256 * kTopkCopies];
   const TopkRow r = topk_row(scores, score_stride, ws, S);
   uint32_t key[8];
-  topk_keys(r.row, topk_vec(scores, score_stride), width, key);
+  topk_keys(r.row, topk_vec(scores, score_stride), width, blockIdx.x * kTopkSeg + 8 * threadIdx.x, key);
   topk_clear(hist);
   __syncthreads();
   uint32_t* mine = hist + (threadIdx.x & (kTopkCopies - 1));
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(1024) void topk_hist_lo_kernel(const uint16_t* __re
   __shared__ uint32_t wtot[4], pick[2];
   const TopkRow r = topk_row(scores, score_stride, ws, S);
   uint32_t key[8];
-  topk_keys(r.row, topk_vec(scores, score_stride), width, key);
+  topk_keys(r.row, topk_vec(scores, score_stride), width, blockIdx.x * kTopkSeg + 8 * threadIdx.x, key);
   topk_clear(hist);
   uint32_t hi, above, prior;
   topk_pick(r.hist_hi, S, (uint32_t)k, 0, wtot, pick, hi, above, prior);  // its barriers also cover the clear
@@ -359,6 +359,49 @@ __global__ __launch_bounds__(1024) void topk_hist_lo_kernel(const uint16_t* __re
   topk_publish(hist, r.hist_lo + (int64_t)blockIdx.x * 256);
 }
 
+// The workgroup's selected positions: lane t holds the 8 V keys of positions e .. of a row (lanes in position order); the
+// keys above T go to their running count from run_gt, T's ties to n_above + theirs from run_eq while that is below
+// n_ties. wtot: 16 u32 of LDS.
+template <int V>
+__device__ __forceinline__ void topk_store(const uint32_t (&key)[V][8], int32_t e, int32_t width, uint32_t T,
+                                           uint32_t n_above, uint32_t n_ties, uint32_t run_gt, uint32_t run_eq,
+                                           uint32_t* wtot, int32_t* __restrict__ orow) {
+  static_assert(1024 * 8 * V <= 0x8000, "the packed counts hold a workgroup's keys");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t cnt = 0;
+#pragma unroll
+  for (int i = 0; i < 8 * V; ++i) {
+    const bool in = e + i < width;
+    cnt += (in && key[i / 8][i % 8] > T) ? 1u : 0u;
+    cnt += (in && key[i / 8][i % 8] == T) ? 0x10000u : 0u;
+  }
+  uint32_t incl = cnt;  // inclusive scan over the wave
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t v = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += v;
+  }
+  if (lane == 63) wtot[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0;  // packed
+#pragma unroll
+  for (int w = 0; w < 16; ++w) before += w < wave ? wtot[w] : 0u;
+  const uint32_t excl = before + incl - cnt;
+  uint32_t o_gt = run_gt + (excl & 0xffffu), o_eq = run_eq + (excl >> 16);
+#pragma unroll
+  for (int i = 0; i < 8 * V; ++i) {
+    if (e + i >= width) continue;
+    const uint32_t x = key[i / 8][i % 8];
+    const int32_t label = bf16_bits_to_f32(key_bits(x)) > -0.5f * kIndexMaskBound ? e + i : -1;  // dead: -1
+    if (x > T) {
+      orow[o_gt++] = label;
+    } else if (x == T) {
+      if (o_eq < n_ties) orow[n_above + o_eq] = label;
+      ++o_eq;
+    }
+  }
+}
+
 __global__ __launch_bounds__(1024) void topk_write_kernel(const uint16_t* __restrict__ scores, int64_t score_stride,
                                                           int32_t width, int32_t S, int32_t k,
                                                           uint32_t* __restrict__ ws, int32_t* __restrict__ out,
@@ -366,7 +409,7 @@ __global__ __launch_bounds__(1024) void topk_write_kernel(const uint16_t* __rest
   __shared__ uint32_t wtot[16], pick[2], before_gt[4], before_eq;
   const TopkRow r = topk_row(scores, score_stride, ws, S);
   uint32_t key[8];
-  topk_keys(r.row, topk_vec(scores, score_stride), width, key);
+  topk_keys(r.row, topk_vec(scores, score_stride), width, blockIdx.x * kTopkSeg + 8 * threadIdx.x, key);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the threshold key T and the count above it, from the two published histograms
   uint32_t hi, above1, lo, n_above, prior_hi, prior_lo;
@@ -385,39 +428,54 @@ __global__ __launch_bounds__(1024) void topk_write_kernel(const uint16_t* __rest
   }
   __syncthreads();
   const uint32_t run_gt = before_gt[0] + before_gt[1] + before_gt[2] + before_gt[3], run_eq = before_eq;
-  const int32_t e = blockIdx.x * kTopkSeg + 8 * tid;
-  uint32_t cnt = 0;
+  uint32_t keys[1][8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const bool in = e + j < width;
-    cnt += (in && key[j] > T) ? 1u : 0u;
-    cnt += (in && key[j] == T) ? 0x10000u : 0u;
-  }
-  uint32_t incl = cnt;  // inclusive scan over the wave
+  for (int j = 0; j < 8; ++j) keys[0][j] = key[j];
+  topk_store(keys, blockIdx.x * kTopkSeg + 8 * tid, width, T, n_above, n_ties, run_gt, run_eq, wtot,
+             out + (int64_t)blockIdx.y * out_stride);
+}
+
+// A whole row in one workgroup, 8 V consecutive scores a lane, its histograms in LDS: one launch instead of three for rows
+// of up to kTopkRowVecs * 8192 scores, where launches and round trips bound the three (graph replays, 1 / 16 rows: of
+// 2048 scores 11.7 / 12.6 -> 7.2 / 7.3 us, 8192 12.1 / 13.1 -> 7.5 / 7.7, 16384 12.7 / 13.4 -> 9.8 / 10.0). Longer rows
+// take the segments' workgroups: at V = 4 one of 20000 took 15.5 us here and 12.7 there.
+template <int V>
+__global__ __launch_bounds__(1024) void topk_row_kernel(const uint16_t* __restrict__ scores, int64_t score_stride,
+                                                        int32_t width, int32_t k, int32_t* __restrict__ out,
+                                                        int64_t out_stride) {
+  __shared__ uint32_t hist[256 * kTopkCopies], folded[256];
+  __shared__ uint32_t wtot[16], pick[2];
+  const int tid = threadIdx.x;
+  const uint16_t* row = scores + (int64_t)blockIdx.y * score_stride;
+  const int32_t e = 8 * V * tid;
+  uint32_t key[V][8];
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += v;
-  }
-  if (lane == 63) wtot[wave] = incl;
+  for (int v = 0; v < V; ++v) topk_keys(row, topk_vec(scores, score_stride), width, e + 8 * v, key[v]);
+  uint32_t* mine = hist + (tid & (kTopkCopies - 1));
+  uint32_t hi, above1, lo, n_above, prior;
+  topk_clear(hist);
   __syncthreads();
-  uint32_t before = 0;  // packed: inside one segment each count is at most kTopkSeg
 #pragma unroll
-  for (int w = 0; w < 16; ++w) before += w < wave ? wtot[w] : 0u;
-  const uint32_t excl = before + incl - cnt;
-  uint32_t o_gt = run_gt + (excl & 0xffffu), o_eq = run_eq + (excl >> 16);
-  int32_t* orow = out + (int64_t)blockIdx.y * out_stride;
+  for (int v = 0; v < V; ++v)
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    if (e + j >= width) continue;
-    const int32_t label = bf16_bits_to_f32(key_bits(key[j])) > -0.5f * kIndexMaskBound ? e + j : -1;  // dead: -1
-    if (key[j] > T) {
-      orow[o_gt++] = label;
-    } else if (key[j] == T) {
-      if (o_eq < n_ties) orow[n_above + o_eq] = label;
-      ++o_eq;
-    }
-  }
+    for (int j = 0; j < 8; ++j)
+      if (e + 8 * v + j < width) atomicAdd(&mine[(key[v][j] >> 8) * kTopkCopies], 1u);
+  __syncthreads();
+  topk_publish(hist, folded);
+  __syncthreads();
+  topk_clear(hist);
+  topk_pick(folded, 1, (uint32_t)k, 0, wtot, pick, hi, above1, prior);  // its barriers also cover the clear
+#pragma unroll
+  for (int v = 0; v < V; ++v)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (e + 8 * v + j < width && (key[v][j] >> 8) == hi) atomicAdd(&mine[(key[v][j] & 0xffu) * kTopkCopies], 1u);
+  __syncthreads();
+  topk_publish(hist, folded);
+  __syncthreads();
+  topk_pick(folded, 1, (uint32_t)k, above1, wtot, pick, lo, n_above, prior);
+  topk_store(key, e, width, (hi << 8) | lo, n_above, (uint32_t)k - n_above, 0u, 0u, wtot,
+             out + (int64_t)blockIdx.y * out_stride);
 }
 
 // e4m3fn(clamp(key, +-448)) rows into an index-key cache; one thread per 8 elements, out-of-cache slots skipped.
@@ -519,11 +577,15 @@ int sna_topk_positions(const void* scores, int64_t score_stride, int32_t B, int3
   const uint16_t* sc = (const uint16_t*)scores;
   uint32_t* ws = (uint32_t*)workspace;
   hipStream_t st = (hipStream_t)stream;
+  if (S <= kTopkRowVecs) {
+    const dim3 rows(1, (unsigned)B);
+    if (S == 1) hipLaunchKernelGGL((topk_row_kernel<1>), rows, block, 0, st, sc, score_stride, width, k, out, out_stride);
+    else hipLaunchKernelGGL((topk_row_kernel<2>), rows, block, 0, st, sc, score_stride, width, k, out, out_stride);
+    return check_launch("topk_positions");
+  }
   hipLaunchKernelGGL(topk_hist_hi_kernel, grid, block, 0, st, sc, score_stride, width, S, ws);
-  hipLaunchKernelGGL(topk_hist_lo_kernel, grid, block, 0, st, sc, score_stride, width, S, k,
-                        ws);
-  hipLaunchKernelGGL(topk_write_kernel, grid, block, 0, st, sc, score_stride, width, S, k, ws, out,
-                        out_stride);
+  hipLaunchKernelGGL(topk_hist_lo_kernel, grid, block, 0, st, sc, score_stride, width, S, k, ws);
+  hipLaunchKernelGGL(topk_write_kernel, grid, block, 0, st, sc, score_stride, width, S, k, ws, out, out_stride);
   return check_launch("topk_positions");
 }
 

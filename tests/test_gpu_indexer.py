@@ -102,6 +102,29 @@ def test_topk_positions_exact(name, seed, B, N, k):
         assert set(got[b].tolist()) == _deterministic_topk(s[b], k)
 
 
+@pytest.mark.parametrize("N,k,stride", [(1, 1, 1), (9, 9, 9), (8191, 2048, 8191), (8193, 1, 8193), (8200, 8200, 8208),
+                                        (16383, 2048, 16391), (16384, 16384, 16384), (16385, 2048, 16392)])
+def test_topk_rows_around_one_workgroup(N, k, stride):
+    """Rows at the edges of one workgroup's 8 and 16 scores a lane, strided rows with and without 16-byte alignment:
+    random scores with ties, one row of a single value, one of dead keys but one, infinities among them."""
+    announce(f"topk rows N={N} k={k} stride={stride}")
+    g = torch.Generator().manual_seed(N)
+    s = torch.full((4, stride), 9e9).to(torch.bfloat16)  # past the row: must not be selected
+    s[:, :N] = (torch.randint(-300, 300, (4, N), generator=g).float() / 16).to(torch.bfloat16)
+    s[1, :N] = -2.5
+    s[2, :N] = -1e30
+    s[2, N // 2] = 1.0
+    s[3, 0], s[3, N - 1] = -float("inf"), float("inf")
+    got = ops.topk_positions(s.to(DEV)[:, :N], k).cpu()
+    for b in range(4):
+        assert sorted(got[b].tolist()) == sorted(_deterministic_list(s[b, :N], k))
+
+
+def _deterministic_list(row, k):
+    r = row.float().tolist()
+    return [e if r[e] > -5e29 else -1 for e in sorted(range(len(r)), key=lambda e: (-r[e], e))[:k]]
+
+
 def test_scores_then_topk_select_every_clear_winner():
     """GPU scores then GPU top-k: every key whose oracle score clears the oracle's k-th value by more than two bf16
     roundings is selected (the scores may differ by one rounding, so the threshold's neighbourhood may differ)."""
