@@ -159,7 +159,7 @@ int sna_kv_store_dsa(const void *rows, const int64_t *slots, int64_t n_tokens, f
  *
  * MLA and DSA (kinds 1, 2): a stream split. Row b's keys (paged: the seq_len - 1 prior positions; sparse: the index
  * list) form ceil(keys / 16) tiles (at least 1), the rows' tiles are laid end to end, and workgroup w takes tiles
- * [cta_start[w], cta_start[w + 1]) of that sequence: n_ctas workgroups (one per CU) of equal tile counts, each
+ * [cta_start[w], cta_start[w + 1]) of that sequence: n_ctas workgroups (at most one per CU) of equal tile counts, each
  * starting in row cta_row[w] at tile cta_off[w] of that row. A workgroup whose range holds a whole row writes its
  * output; a row split over several workgroups is merged inside the same launch (its workgroups publish partials and
  * the last to arrive, with those still waiting for it, merges them), so one launch is the whole decode. row_keys[b] is

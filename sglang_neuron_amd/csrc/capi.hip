@@ -28,13 +28,13 @@ int32_t host_splits(int32_t seq_len, int32_t window, int32_t tile, int32_t split
 int32_t host_tiles(int32_t seq_len, int32_t window, int32_t tile) { return host_splits(seq_len, window, tile, 1); }
 
 // The MLA / DSA stream split: every row's key tiles (at least one, so a row with no prior key still has a workgroup
-// to attend its own row) laid end to end, cut into n_ctas ranges of equal tile counts. A workgroup runs per CU (the
-// kernel's LDS holds one), so n_ctas is the CU count over the head groups, fewer when there are fewer tiles; a sparse workgroup resolves at
-// most kMlaMaxSplitKeys indices in LDS, and sparse rows are latency-bound gathers, so a sparse plan aims for
+// to attend its own row) laid end to end, cut into n_ctas ranges of equal tile counts. A CU holds one workgroup (the
+// kernel's LDS), so n_ctas is at most the CU count over the head groups, and at most what the rows are worth: paged rows
+// stream_pieces each, summed over the batch (the longest rows may take more). A sparse workgroup resolves at most
+// kMlaMaxSplitKeys indices in LDS, and sparse rows are latency-bound gathers, so a sparse plan aims for
 // kSparseTilesPerCta tiles per workgroup (about three per wave: every tile's gathers go out at once). Measured on
 // cfg5's 2048-index rows, 11 tiles (~12 workgroups a row) beat 8 (16 a row) by 0.5 us at 16 rows and 0.3 us at 8,
-// and tie at 4; 12 tiles and 8 workgroups a row were slower. A paged row takes at most stream_pieces workgroups on
-// average over the batch.
+// and tie at 4; 12 tiles and 8 workgroups a row were slower.
 constexpr int64_t kSparseTilesPerCta = 11;
 int plan_stream(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32_t max_seq_len, int32_t n_keys_per_row,
                 int32_t groups, int32_t num_cus, sna_split_plan* plan) {
