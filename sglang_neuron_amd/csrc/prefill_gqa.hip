@@ -85,6 +85,9 @@ constexpr int kPrefillSlots = 512;
 constexpr int kPrefillSplitBlocks = 256;
 constexpr int kPrefillMinSplit = 8;
 constexpr int kPrefillNoSplit = 16;
+// The most tiles of a query block of a launch that splits (prefill_item's exact divisions hold below 2^17): a table that
+// can name more keys runs unsplit, which reads any length.
+constexpr int kPrefillSplitMaxTiles = (1 << 17) - 1;
 
 template <int D, int ESZ>  // ESZ: bytes per K/V element (1: e4m3fn, 2: bf16)
 struct PrefillGeo {
@@ -153,7 +156,8 @@ __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32
         const int32_t rr = div_small(p, a.qblocks, rq);
         const int32_t S = a.q_start[rr + 1] - a.q_start[rr];
         const PrefillBlock b = prefill_block(a, S, a.prior[rr], p - rr * a.qblocks);
-        tiles[i] = b.nq > 0 ? min(b.t1 - b.t0, (1 << 17) - 1) : 0;
+        // (held to the launch's bound: a length past the table's keys has only invalid keys there)
+        tiles[i] = b.nq > 0 ? min(b.t1 - b.t0, kPrefillSplitMaxTiles) : 0;
       }
       lane_total += tiles[i];
       lane_max = max(lane_max, tiles[i]);
@@ -187,7 +191,7 @@ __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32
       per_head += part;
       blocks += __popcll(__ballot(tiles[i] > 0));
     }
-  // tenths of a microsecond, in 64 bits (a row may span 2^17 tiles)
+  // tenths of a microsecond, in 64 bits
   const int64_t whole = (int64_t)mx * 13;  // (at most one block a CU)
   const int64_t cut = (int64_t)st * (per_head * a.G > kPrefillSlots / 2 ? 20 : 13) + 50 + per_head * a.G * 10 / 32;
   if (cut >= whole) {
@@ -658,10 +662,10 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a, boo
 
 // The workgroups of a split launch: 0 where the launch's own query blocks are more than one a CU (they reach the rate
 // that the power limit allows by themselves: 352 blocks of up to 137 tiles took 170 us whole, 186 in a split launch; 376
-// of up to 24 tiles 41 and 49) or too short.
+// of up to 24 tiles 41 and 49), too short, or past what the split counts.
 static int32_t prefill_split_slots(int64_t qblocks, int32_t R, int32_t G, int64_t bound_tiles) {
   const int64_t base = qblocks * R * G;
-  if (base > kPrefillSplitBlocks || bound_tiles <= kPrefillNoSplit) return 0;
+  if (base > kPrefillSplitBlocks || bound_tiles <= kPrefillNoSplit || bound_tiles > kPrefillSplitMaxTiles) return 0;
   static_assert(kPrefillSplitPairs >= kPrefillSplitBlocks, "a split launch's pairs fit a wave");
   return (int32_t)std::min<int64_t>(kPrefillSlots, base * ((bound_tiles + kPrefillMinSplit - 1) / kPrefillMinSplit));
 }

@@ -245,6 +245,19 @@ def test_mla_plan_takes_sqrt_3_tiles_workgroups_a_row(lib, tiles):
     _check_stream_plan(p, [16 * t for t in tiles], 256)
 
 
+def test_prefill_split_holds_its_tile_counts(lib):
+    """A prefill launch splits its keys only where the kernel's 2^17 - 1 tiles of 64 keys hold every key the table can
+    name (past them it runs unsplit, which reads any length); inside a window only the window's keys count."""
+    widest = ((1 << 17) - 1) * 64 // 16  # pages of 16
+
+    def need(width, window=0, page=16):
+        return lib.sna_prefill_workspace_bytes(1, 16, 1, 1, 64, page, width, window)
+
+    assert need(widest) > 0 and need(widest + 1) == 0
+    assert need(1 << 20) == 0 and need(1 << 14, page=1 << 16) == 0
+    assert need(1 << 20, window=100000) > 0
+
+
 def test_dsa_stream_plan(lib):
     rc, p = _plan(lib, _lib.KIND_DSA, B=16, keys=2048, ctas=1)
     assert rc == 0
