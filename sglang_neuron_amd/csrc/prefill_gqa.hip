@@ -156,8 +156,10 @@ __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32
         const int32_t rr = div_small(p, a.qblocks, rq);
         const int32_t S = a.q_start[rr + 1] - a.q_start[rr];
         const PrefillBlock b = prefill_block(a, S, a.prior[rr], p - rr * a.qblocks);
-        // (held to the launch's bound: a length past the table's keys has only invalid keys there)
-        tiles[i] = b.nq > 0 ? min(b.t1 - b.t0, kPrefillSplitMaxTiles) : 0;
+        // A block with queries has an item, and no length the device may hold makes more than the workspace's: its tiles
+        // are held to the launch's bound (past the table's keys all are invalid) and, for a negative prior, from below
+        // (such a block's item runs no tile, as the unsplit kernel's).
+        tiles[i] = b.nq > 0 ? max(1, min(b.t1 - b.t0, kPrefillSplitMaxTiles)) : 0;
       }
       lane_total += tiles[i];
       lane_max = max(lane_max, tiles[i]);

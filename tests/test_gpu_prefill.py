@@ -191,6 +191,30 @@ def test_prefill_ignores_unused_slots_and_invalid_pages(bf16, prior):
     assert_close_attn(out.cpu(), want, "nan slots")
 
 
+def test_prefill_split_ignores_lengths_it_cannot_hold():
+    """In a launch that splits, a padding request (no token) and one whose prior is below zero (no visible key: its rows
+    are what the unsplit entry writes) leave the other requests' splits and outputs as they are without them."""
+    announce("prefill split padding requests")
+    H, G, d, P = 8, 2, 64, 16
+    q, kc, vc, ks, vs, table, _, _ = _case(41, H=H, G=G, d=d, P=P, priors=(2500, 0, 0), lens=(40, 0, 16))
+    dev = [t.to(DEV) for t in (ks, vs)]
+    q_start = torch.tensor([0, 40, 40, 56], dtype=torch.int32, device=DEV)
+    lib = _lib.load()
+
+    def run(n, priors):
+        R = len(priors)
+        assert lib.sna_prefill_workspace_bytes(R, 40, H, G, d, P, table.shape[1], 0) > 0
+        return ops.prefill_attention(q[:n].to(DEV), kc, vc, table[:R].to(DEV), q_start[:R + 1],
+                                     torch.tensor(priors, dtype=torch.int32, device=DEV), max_q_len=40, sm_scale=0.125,
+                                     k_scale=dev[0], v_scale=dev[1]).cpu()
+
+    alone = run(40, [2500])
+    for low in (-300, -64, -5000):
+        both = run(56, [2500, low, low])
+        assert torch.equal(both[:40], alone), low
+        assert bool(torch.isnan(both[40:].float()).all()), low  # softmax over no key
+
+
 def test_prefill_split_workspace_refusals():
     """A workspace smaller than the split needs, or not 16-byte aligned, is refused before any launch."""
     q, kc, vc, ks, vs, table, q_start, priors = _case(26, H=8, G=2, d=64, P=16, priors=(1900,), lens=(20,))
