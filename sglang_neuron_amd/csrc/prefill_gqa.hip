@@ -435,7 +435,8 @@ void prefill_gqa_kernel(PrefillArgs a) {
       }
   };
   auto mask = [&](int32_t k0, uint32_t pg_ok, f32x16_t (&y)[NSUB]) {
-    const int32_t last = qpos - 8 * g2, first = a.window > 0 ? last - a.window + 1 : INT32_MIN;
+    // (no position is below 0, so neither is a window's first key: `first` does not leave 32 bits for any window)
+    const int32_t last = qpos - 8 * g2, first = a.window > 0 ? max(qpos - a.window + 1, 0) - 8 * g2 : INT32_MIN;
     mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < NSUB; ++u)

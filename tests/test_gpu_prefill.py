@@ -215,6 +215,20 @@ def test_prefill_split_ignores_lengths_it_cannot_hold():
         assert bool(torch.isnan(both[40:].float()).all()), low  # softmax over no key
 
 
+@pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
+@pytest.mark.parametrize("prior", [0, 1500], ids=["whole", "split"])
+def test_prefill_widest_window_is_no_window(bf16, prior):
+    """A window of up to 2^31 - 1 keys holds every key of any row: the outputs are those of no window."""
+    announce(f"prefill widest window bf16={bf16} prior={prior}")
+    H, G, d, P, n = 8, 2, 64, 16, 70
+    q, kc, vc, ks, vs, table, q_start, priors = _case(43, H=H, G=G, d=d, P=P, priors=(prior,), lens=(n,), bf16=bf16)
+    kw = dict(max_q_len=n, sm_scale=0.125, k_scale=None if bf16 else ks.to(DEV), v_scale=None if bf16 else vs.to(DEV))
+    args = (q.to(DEV), kc, vc, table.to(DEV), q_start.to(DEV), priors.to(DEV))
+    none = ops.prefill_attention(*args, **kw)
+    for window in (2**31 - 1, 2**31 - 4, 2**31 - 64, 1 << 20):
+        assert torch.equal(ops.prefill_attention(*args, window=window, **kw), none), window
+
+
 def test_prefill_split_workspace_refusals():
     """A workspace smaller than the split needs, or not 16-byte aligned, is refused before any launch."""
     q, kc, vc, ks, vs, table, q_start, priors = _case(26, H=8, G=2, d=64, P=16, priors=(1900,), lens=(20,))
