@@ -307,9 +307,9 @@ int sna_paged_decode_gqa(const void *q, const void *k_cache, const void *v_cache
  * and the active tokens, token t at position seq_len - n_tokens + t. The tokens are stored (sna_kv_store_mha on `stream`),
  * then token t attends the row's prior keys and the active tokens 0 .. t: a workgroup's tokens in-band at their stored
  * (dequantized) values, earlier ones from the pool, so a row's keys are read once for 16 / group tokens. A window (at
- * least n_tokens) applies to each token. The plan: sna_plan_decode for the B rows, with window + n_tokens - 1 when there
- * is a window and num_kv_heads * ceil(n_tokens / (16 / group)) (under a window num_kv_heads * n_tokens) workgroups an
- * item; the workspace: sna_decode_workspace_bytes(plan, n_tokens * num_q_heads, head_dim).
+ * least n_tokens) applies to each token. The plan: sna_plan_decode for the B rows, with window + n_tokens - 1 (at most
+ * 2^31 - 1) when there is a window and num_kv_heads * ceil(n_tokens / (16 / group)) (under a window num_kv_heads *
+ * n_tokens) workgroups an item; the workspace: sna_decode_workspace_bytes(plan, n_tokens * num_q_heads, head_dim).
  * Replaces: _torch_attention_decode with X [B, S, Hd] (ops/attention/attention_decode.py:226-300). */
 int sna_paged_decode_gqa_multi(const void *q, void *k_cache, void *v_cache, const float *k_scale, const float *v_scale,
                                const int32_t *block_table, int64_t table_stride, int32_t table_width,

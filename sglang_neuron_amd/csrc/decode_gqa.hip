@@ -838,7 +838,7 @@ int decode_gqa(const char* what, const void* q, const void* k_cache, const void*
   a.tpi = window > 0 ? 1 : std::min(16 / group, S);
   a.chunks = (S + a.tpi - 1) / a.tpi;
   a.token_window = window;
-  a.window = window > 0 ? window + S - 1 : 0;
+  a.window = window > 0 ? (int32_t)std::min<int64_t>((int64_t)window + S - 1, INT32_MAX) : 0;
   a.sm_scale = sm_scale;
   a.split_tiles = plan->split_tiles;
   a.dev_split = plan->device_split;

@@ -587,7 +587,8 @@ def paged_decode_gqa_multi(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_ta
     # a row's workgroups per (split, KV head): 16 / group tokens each, one under a window
     chunks = S if window > 0 else -(-S // max(1, 16 // (H // G)))
     plan = plan_decode(_lib.KIND_GQA, B, host_seq_lens=hl, max_seq_len=table.shape[1] * P,
-                       window=window + S - 1 if window > 0 else 0, ctas_per_item=G * chunks, num_cus=_num_cus(dev))
+                       window=min(window + S - 1, 2**31 - 1) if window > 0 else 0, ctas_per_item=G * chunks,
+                       num_cus=_num_cus(dev))
     ws = torch.empty(max(workspace_bytes(plan, H * S, d), 16), dtype=torch.uint8, device=dev)
     rc = _lib.load().sna_paged_decode_gqa_multi(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), _ptr(table), table.stride(0),

@@ -302,3 +302,23 @@ def test_gqa_multi_device_lengths_and_padding_rows():
     pad = ops.paged_decode_gqa_multi(qd, kcd, vcd, td, ld, knd, vnd, **kw)
     torch.cuda.synchronize()
     assert torch.equal(pad[:2], bound[:2]) and bool(torch.isfinite(pad).all())
+
+
+def test_gqa_multi_widest_window():
+    """A window of up to 2^31 - 1 keys holds every key of any row: the outputs are those of a window past the rows."""
+    from sglang_neuron_amd import ops
+
+    B, S, H, G, d, P = 2, 4, 8, 2, 64, 16
+    lens = [90, 700]
+    q, kc, vc, table, kn, vn, slots = [t.cuda() for t in _multi_inputs(7, B, S, H, G, d, P, lens)]
+    announce("gqa multi widest window")
+    ld = torch.tensor(lens, dtype=torch.int32, device="cuda")
+
+    def run(window, **kw):
+        return ops.paged_decode_gqa_multi(q, kc, vc, table, ld, kn, vn, sm_scale=0.125, new_slots=slots, window=window, **kw)
+
+    for kw in ({"host_seq_lens": lens}, {}):
+        want = run(1 << 20, **kw)
+        assert bool(torch.isfinite(want).all())
+        for window in (2**31 - 1, 2**31 - 3, 2**31 - S):
+            assert torch.equal(run(window, **kw), want), (window, sorted(kw))
