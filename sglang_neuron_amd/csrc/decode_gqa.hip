@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "sna_device.h"
 #include "sna_host.h"
@@ -65,12 +66,17 @@ struct GqaArgs {
   float* ws_ml;  // [B, max_splits, H, 2]  reference max (log2 domain) and softmax sum
   int32_t* ws_st;  // a device split's split size, written by the decode launch for its combine (after ws_ml)
   uint16_t* out;
-  // S active tokens per row (MULTI launches; 1 otherwise): q, k_new, v_new, out and the partials have B * S rows, row
-  // b * S + t for token t of row b at position seq_len - S + t. A workgroup's 16 columns hold `tpi` tokens' group heads
-  // (one token's under a window), so a row takes `chunks` workgroups per (split, KV head). `window` then spans all S
-  // tokens' windows (token_window is one token's): every chunk of a row runs the same splits.
+};
+
+// S active tokens per row (MULTI launches): q, k_new, v_new, out and the partials have B * S rows, row b * S + t for token
+// t of row b at position seq_len - S + t. A workgroup's 16 columns hold `tpi` tokens' group heads (one token's under a
+// window), so a row takes `chunks` workgroups per (split, KV head). `window` then spans all S tokens' windows
+// (token_window is one token's): every chunk of a row runs the same splits.
+struct GqaMultiArgs : GqaArgs {
   int32_t S, tpi, chunks, token_window;
 };
+template <bool MULTI>
+using GqaArgsOf = std::conditional_t<MULTI, GqaMultiArgs, GqaArgs>;
 
 // The splits this launch runs for row b: its entries in the plan's item map (counted on the host), or (no map: items
 // located from seq_lens) the device length's split count, with split size st, up to the plan's.
@@ -191,7 +197,7 @@ struct GqaTile {
 
 template <int D, bool FP8, int WAVES, bool FINAL, int DEPTH, bool MULTI>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
-void gqa_decode_kernel(GqaArgs a) {
+void gqa_decode_kernel(GqaArgsOf<MULTI> a) {
   using Tile = GqaTile<D, FP8>;
   constexpr int ESZ = Tile::ESZ;
   constexpr int STEPS = D / 32;  // QK MFMA steps
@@ -209,9 +215,12 @@ void gqa_decode_kernel(GqaArgs a) {
   const int g = blockIdx.y;
   // the split item; MULTI: eight items' first chunks, then their second ones, ...: an item's chunks run on one XCD, whose
   // L2 they share (the grid's width is a multiple of 8)
-  const int32_t item = MULTI ? (int32_t)(blockIdx.x / (8 * a.chunks) * 8 + blockIdx.x % 8) : (int32_t)blockIdx.x;
-  const int32_t chunk = MULTI ? (int32_t)(blockIdx.x / 8 % a.chunks) : 0;
-  if (MULTI && item >= a.n_work) return;
+  int32_t item = (int32_t)blockIdx.x, chunk = 0;
+  if constexpr (MULTI) {
+    item = (int32_t)(blockIdx.x / (8 * a.chunks) * 8 + blockIdx.x % 8);
+    chunk = (int32_t)(blockIdx.x / 8 % a.chunks);
+    if (item >= a.n_work) return;
+  }
 
   int32_t b, split, st, L = 0;
   if (a.dev_split) {  // the split size and the item, from the device's lengths
@@ -234,10 +243,9 @@ void gqa_decode_kernel(GqaArgs a) {
   // write leaves the workspace
   if (b < 0 || b >= a.B || split >= max(a.max_splits, 1)) return;
   // the workgroup's columns: column c is query head g * group + c % group of token t0 + c / group (one token: heads only)
-  const int32_t t0 = MULTI ? chunk * a.tpi : 0;
-  const int32_t ntok = MULTI ? min(a.tpi, a.S - t0) : 1;
+  int32_t t0 = 0, ntok = 1, row0 = b;  // row0: the first token's row in q, k_new, v_new and out
+  if constexpr (MULTI) t0 = chunk * a.tpi, ntok = min(a.tpi, a.S - t0), row0 = b * a.S + t0;
   const int32_t cols = ntok * a.group;
-  const int32_t row0 = MULTI ? b * a.S + t0 : b;  // the first token's row in q, k_new, v_new and out
   auto col_token = [&](int32_t c) -> int32_t { return MULTI ? c / a.group : 0; };
   auto col_row = [&](int32_t c) -> int64_t {  // the column's (row, head) in q and out
     const int32_t t = col_token(c);
@@ -515,45 +523,55 @@ void gqa_decode_kernel(GqaArgs a) {
 
   // ---- the step's own token (operands loaded before the tile loop) ----
   __shared__ float sm_kn[OWN_T * D], sm_vn[OWN_T * D], sm_sn[16 * OWN_T];
-  if (own) {
-#pragma unroll
-    for (int i = 0; i < OWN_E; ++i) {
-      const int e = tid + 64 * WAVES * i;
-      if (e >= (MULTI ? ntok * D : D)) break;
-      const uint32_t kb = own_kb[i], vb = own_vb[i];
-      const int64_t dst = own_dst;
-      float kd, vd;
-      if constexpr (FP8) {
-        const uint32_t kq = a.mul_scale ? quantize_e4m3fn_mul(kb, kstored) : quantize_e4m3fn(kb, kscale);
-        const uint32_t vq = a.mul_scale ? quantize_e4m3fn_mul(vb, vstored) : quantize_e4m3fn(vb, vscale);
-        kd = e4m3fn_to_f32(kq) * kscale;
-        vd = e4m3fn_to_f32(vq) * vscale;
-        if (dst >= 0) {
-          a.k_cache[dst] = (uint8_t)kq;
-          a.v_cache[dst] = (uint8_t)vq;
-        }
-      } else {
-        kd = bf16_bits_to_f32(kb);
-        vd = bf16_bits_to_f32(vb);
-        if (dst >= 0) {
-          reinterpret_cast<uint16_t*>(a.k_cache)[dst] = (uint16_t)kb;
-          reinterpret_cast<uint16_t*>(a.v_cache)[dst] = (uint16_t)vb;
-        }
+  // element e of the workgroup's tokens: its dequantized values into LDS, its pool bytes stored (dst >= 0)
+  auto own_element = [&](int e, uint32_t kb, uint32_t vb, int64_t dst) {
+    float kd, vd;
+    if constexpr (FP8) {
+      const uint32_t kq = a.mul_scale ? quantize_e4m3fn_mul(kb, kstored) : quantize_e4m3fn(kb, kscale);
+      const uint32_t vq = a.mul_scale ? quantize_e4m3fn_mul(vb, vstored) : quantize_e4m3fn(vb, vscale);
+      kd = e4m3fn_to_f32(kq) * kscale;
+      vd = e4m3fn_to_f32(vq) * vscale;
+      if (dst >= 0) {
+        a.k_cache[dst] = (uint8_t)kq;
+        a.v_cache[dst] = (uint8_t)vq;
       }
-      sm_kn[e] = kd;
-      sm_vn[e] = vd;
+    } else {
+      kd = bf16_bits_to_f32(kb);
+      vd = bf16_bits_to_f32(vb);
+      if (dst >= 0) {
+        reinterpret_cast<uint16_t*>(a.k_cache)[dst] = (uint16_t)kb;
+        reinterpret_cast<uint16_t*>(a.v_cache)[dst] = (uint16_t)vb;
+      }
+    }
+    sm_kn[e] = kd;
+    sm_vn[e] = vd;
+  };
+  if (own) {
+    if constexpr (MULTI) {
+#pragma unroll
+      for (int i = 0; i < OWN_E; ++i) {
+        const int e = tid + 64 * WAVES * i;
+        if (e < ntok * D) own_element(e, own_kb[i], own_vb[i], -1);
+      }
+    } else if (tid < D) {
+      own_element(tid, own_kb[0], own_vb[0], own_dst);
     }
     __syncthreads();
 #pragma unroll
     for (int jj = 0; jj < OWN_J; ++jj) {
       const int j = wave + WAVES * jj;  // uniform
       if (j >= cols) break;
-      for (int u = 0; u <= col_token(j); ++u) {  // the workgroup's tokens up to the column's own
+      auto score = [&](int u) {
         float s = 0.0f;
 #pragma unroll
         for (int v = 0; v < D / 64; ++v) s += own_q[jj][v] * sm_kn[u * D + lane + 64 * v];
         s = wave_sum(s);
         if (lane == 0) sm_sn[j * OWN_T + u] = s * a.sm_scale * kLog2e;
+      };
+      if constexpr (MULTI) {
+        for (int u = 0; u <= col_token(j); ++u) score(u);  // the workgroup's tokens up to the column's own
+      } else {
+        score(0);
       }
     }
   }
@@ -579,8 +597,12 @@ void gqa_decode_kernel(GqaArgs a) {
     const int j = idx / D, d = idx % D;
     const int32_t t = col_token(j), h = g * a.group + j - t * a.group;
     float M = -INFINITY;
-    if (own)
-      for (int u = 0; u <= t; ++u) M = fmaxf(M, sm_sn[j * OWN_T + u]);
+    if constexpr (MULTI) {
+      if (own)
+        for (int u = 0; u <= t; ++u) M = fmaxf(M, sm_sn[j * OWN_T + u]);
+    } else {
+      M = own ? sm_sn[j] : -INFINITY;
+    }
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) M = fmaxf(M, sm_m[w][j]);
     float o = 0.0f, l = 0.0f;
@@ -592,7 +614,7 @@ void gqa_decode_kernel(GqaArgs a) {
     }
     o *= vscale;
     if (own) {
-      for (int u = 0; u <= t; ++u) {
+      for (int u = 0; u <= (MULTI ? t : 0); ++u) {
         const float e = __builtin_amdgcn_exp2f(sm_sn[j * OWN_T + u] - M);
         o += e * sm_vn[u * D + d];
         l += e;
@@ -617,7 +639,7 @@ void gqa_decode_kernel(GqaArgs a) {
 // head dims D / 64 * i .. + D / 64. The partials stream in chunks of 16 splits, each chunk's loads all in flight
 // together (the first before the weights are known).
 template <int D, bool MULTI>
-__global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
+__global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgsOf<MULTI> a) {
   constexpr int V = D / 64;
   constexpr int CH = 16;
   const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
@@ -635,7 +657,8 @@ __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
     for (int v = 0; v < V; ++v) x[k][v] = k < S ? ob[k * sstride + v] : 0.0f;
   float2 ml = make_float2(-INFINITY, 0.0f);
   if (lane < S) ml = *reinterpret_cast<const float2*>(a.ws_ml + (row0 + (int64_t)lane * a.H) * 2);
-  const int32_t br = MULTI ? b / a.S : b;  // the row of seq_lens (S tokens a row)
+  int32_t br = b;  // the row of seq_lens (MULTI: S tokens a row)
+  if constexpr (MULTI) br = b / a.S;
   const int32_t n = min(launched_splits(a, br, ld_const(a.seq_lens + br), a.dev_split ? *a.ws_st : a.split_tiles), S);
   if (n == 0) return;  // a row with no prior key: the lone-token kernel writes it
   const float m = lane < n ? ml.x : -INFINITY, l = lane < n ? ml.y : 0.0f;
@@ -670,10 +693,11 @@ __global__ __launch_bounds__(64) void gqa_combine_kernel(GqaArgs a) {
 
 // Rows with no split at all (seq_len 1) get their output from this pass: only the own token (and the sink).
 template <int D, bool FP8, bool MULTI>
-__global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgs a) {
+__global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgsOf<MULTI> a) {
   const int b = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
   // any split size counts the row's splits as nonzero iff it has a prior key
-  const int32_t br = MULTI ? b / a.S : b;  // (S tokens a row)
+  int32_t br = b;
+  if constexpr (MULTI) br = b / a.S;  // (S tokens a row)
   if (launched_splits(a, br, a.seq_lens[br], a.split_tiles) > 0) return;
   __shared__ float sm_kn[D], sm_vn[D];
   const float kstored = FP8 ? a.k_scale[g] : 1.0f, vstored = FP8 ? a.v_scale[g] : 1.0f;
@@ -726,9 +750,11 @@ __global__ __launch_bounds__(128) void gqa_lone_token_kernel(GqaArgs a) {
 }
 
 template <int D, bool FP8, bool MULTI>
-static void launch_gqa(const GqaArgs& a, bool any_lone, hipStream_t s) {
+static void launch_gqa(const GqaArgsOf<MULTI>& a, bool any_lone, hipStream_t s) {
+  int32_t S = 1, chunks = 1;
+  if constexpr (MULTI) S = a.S, chunks = a.chunks;
   if (a.n_work > 0) {
-    const dim3 grid(MULTI ? (a.n_work + 7) / 8 * 8 * a.chunks : a.n_work, a.G);
+    const dim3 grid(MULTI ? (a.n_work + 7) / 8 * 8 * chunks : a.n_work, a.G);
     // two register tiles per wave whatever the plan's shape (rings of 3 and 4 measured 1% and 2% slower on the cfg2
     // and cfg4 batches: fewer loads outstanding per wave stream faster). Splits of 5 to 64 tiles run on 8 waves, so
     // a wave walks half as many tiles one after the other (cfg4-swa's 5-tile rows 7.98 -> 6.45 us, cfg4's 48-tile
@@ -737,7 +763,7 @@ static void launch_gqa(const GqaArgs& a, bool any_lone, hipStream_t s) {
     // two (16 rows of 500-2000 keys, 32 / 8 heads, FP8: 21.1 us on 8 waves, 16.8 on 4; one row of 32000 25.2 and 21.9;
     // 16 rows of 1000-8000 35.8 and 32.7). cfg2's whole 128-tile rows run on 4 (91 against 94).
     const bool eight = a.split_tiles > 4 && a.split_tiles <= 64 &&
-                       (D == 64 || (int64_t)a.n_work * a.chunks * a.G <= 256);
+                       (D == 64 || (int64_t)a.n_work * chunks * a.G <= 256);
     if (a.max_splits <= 1) {
       if (eight) hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 8, true, 2, MULTI>), grid, dim3(512), 0, s, a);
       else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, true, 2, MULTI>), grid, dim3(256), 0, s, a);
@@ -746,12 +772,12 @@ static void launch_gqa(const GqaArgs& a, bool any_lone, hipStream_t s) {
       else hipLaunchKernelGGL((gqa_decode_kernel<D, FP8, 4, false, 2, MULTI>), grid, dim3(256), 0, s, a);
     }
   }
-  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D, MULTI>), dim3(a.B * a.S, a.H), dim3(64), 0, s, a);
-  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8, MULTI>), dim3(a.B * a.S, a.G), dim3(128), 0, s, a);
+  if (a.max_splits > 1) hipLaunchKernelGGL((gqa_combine_kernel<D, MULTI>), dim3(a.B * S, a.H), dim3(64), 0, s, a);
+  if (any_lone) hipLaunchKernelGGL((gqa_lone_token_kernel<D, FP8, MULTI>), dim3(a.B * S, a.G), dim3(128), 0, s, a);
 }
 
 template <int D, bool FP8>
-static void launch_gqa_tokens(const GqaArgs& a, bool any_lone, hipStream_t s) {
+static void launch_gqa_tokens(const GqaMultiArgs& a, bool any_lone, hipStream_t s) {
   if (a.S > 1) launch_gqa<D, FP8, true>(a, any_lone, s);
   else launch_gqa<D, FP8, false>(a, any_lone, s);
 }
@@ -813,7 +839,7 @@ int decode_gqa(const char* what, const void* q, const void* k_cache, const void*
                 (long long)workspace_bytes, (long long)need);
   if (num_q_heads > 65535) return fail(SNA_ERR_INVALID_ARGUMENT, "%s: grid too large", what);
 
-  GqaArgs a;
+  GqaMultiArgs a;
   a.q = (const uint16_t*)q;
   a.k_cache = (uint8_t*)k_cache;
   a.v_cache = (uint8_t*)v_cache;
