@@ -29,8 +29,8 @@ int32_t host_tiles(int32_t seq_len, int32_t window, int32_t tile) { return host_
 
 // The MLA / DSA stream split: every row's key tiles (at least one, so a row with no prior key still has a workgroup
 // to attend its own row) laid end to end, cut into n_ctas ranges of equal tile counts. A CU holds one workgroup (the
-// kernel's LDS), so n_ctas is at most the CU count over the head groups, and at most what the rows are worth: paged rows
-// stream_pieces each, summed over the batch (the longest rows may take more). A sparse workgroup resolves at most
+// kernel's LDS), so n_ctas is at most the CU count over the head groups, and at most what the rows are worth: paged rows of
+// a batch of up to kStreamWorthRows stream_pieces each, summed (the longest rows may take more). A sparse workgroup resolves at most
 // kMlaMaxSplitKeys indices in LDS, and sparse rows are latency-bound gathers, so a sparse plan aims for
 // kSparseTilesPerCta tiles per workgroup (about three per wave: every tile's gathers go out at once). Measured on
 // cfg5's 2048-index rows, 11 tiles (~12 workgroups a row) beat 8 (16 a row) by 0.5 us at 16 rows and 0.3 us at 8,
@@ -88,9 +88,10 @@ int plan_stream(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32_t m
   const int32_t cus = std::max(1, std::min((num_cus > 0 ? num_cus : 256) / groups, SNA_MAX_CTAS));
   int64_t n = 0;
   if (total > 0) {
-    int64_t pieces = 0;
-    for (int32_t b = 0; b < B; ++b) pieces += stream_pieces(std::max((plan->row_keys[b] + 15) / 16, 1));
-    if (max_tiles <= kStreamWholeTiles) pieces = B;
+    int64_t pieces = B <= kStreamWorthRows ? 0 : total;
+    if (B <= kStreamWorthRows)
+      for (int32_t b = 0; b < B; ++b) pieces += stream_pieces(std::max((plan->row_keys[b] + 15) / 16, 1), B);
+    if (max_tiles <= stream_whole_tiles(B)) pieces = B;
     n = kind == 1 ? std::min<int64_t>(cus, pieces)
                   : std::min<int64_t>(cus, std::max<int64_t>((total + kSparseTilesPerCta - 1) / kSparseTilesPerCta, 1));
     // a sparse range holds at most kSparseCap tiles: equal ranges need ceil(total / cap) of them, and whole rows
@@ -177,7 +178,6 @@ int plan_stream(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32_t m
   plan->n_ctas = (int32_t)n;
   plan->total_tiles = (int32_t)total;
   plan->wait_polls = kStreamWaitPolls;
-  (void)max_tiles;
   return SNA_OK;
 }
 

@@ -249,9 +249,11 @@ __device__ __forceinline__ void wave_incl_scan4(uint32_t (&v)[4]) {
 // table's width and the stream's 65535 tiles per row) into keys[b]; the ranges' starts into cs[w] (cs[w] = the
 // stream's end for w at or past the split's n, and cs[256] too); row << 16 | tile offset into cro[w]; n into *n_out.
 // With a workgroup for every row (B <= n, n = min(launched workgroups, the rows' stream_pieces)) rows are apportioned
-// whole: the least piece length T with sum_b ceil(tiles_b / T) <= n is found by bisection, and row b is cut into ceil(tiles_b / T)
-// equal pieces (the same longest piece as the host planner's greedy apportionment, within a tile); otherwise the
-// stream is cut into n equal ranges. tmp: 5 x 256 words of LDS scratch.
+// whole: the least piece length T with sum_b ceil(tiles_b / T) <= n is found by bisection (about 0.25 us a step), and row b
+// is cut into ceil(tiles_b / T) equal pieces (the same longest piece as the host planner's greedy apportionment, within a
+// tile), at least stream_least(B) of them where the launch has the workgroups; otherwise the stream is cut into n equal
+// ranges. A batch whose longest row has at most kStreamWholeTiles tiles is not cut (whatever B: of 12 tiles, 24 rows took
+// 17.8 us whole in a device split and 16.9 in six pieces, bf16, FP8 19.0 and 18.6). tmp: 5 x 256 words of LDS scratch.
 __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int32_t* keys, int32_t* n_out,
                              uint32_t* tmp) {
   const int lane = threadIdx.x & 63;
@@ -269,7 +271,7 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
     }
     first[i] = tiles[i];
     mx = max(mx, tiles[i]);
-    worth += (uint32_t)stream_pieces((int32_t)tiles[i]);
+    if (B <= kStreamWorthRows && 64 * i < B) worth += (uint32_t)stream_pieces((int32_t)tiles[i], B);  // (uniform branch)
   }
   wave_incl_scan4(first);
   uint32_t total = 0;
@@ -280,7 +282,10 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
     total += part;
   }
   mx = (uint32_t)wave_max((float)mx);
-  const uint32_t n = min((uint32_t)gridDim.x, mx <= kStreamWholeTiles ? (uint32_t)B : (uint32_t)wave_sum((float)worth));
+  uint32_t n = total;
+  // (up to 12 tiles, more than 16 rows: the CUs give the pieces their worth would, without a bisection step)
+  if (B <= 16 || (B <= kStreamWorthRows && mx > 12)) n = (uint32_t)wave_sum((float)worth);
+  n = min((uint32_t)gridDim.x, mx <= (uint32_t)kStreamWholeTiles ? (uint32_t)B : n);
   uint32_t* t_first = tmp;
   uint32_t* t_tiles = tmp + 256;
   uint32_t* t_pieces = tmp + 512;
@@ -312,9 +317,12 @@ __device__ void device_split(const MlaArgs& a, uint32_t* cs, uint32_t* cro, int3
       else lo = mid + 1;
     }
     const float rt = 1.0f / (float)lo;
+    // (where the launch has workgroups for n and every row's least)
+    const uint32_t least = mx > (uint32_t)kStreamWholeTiles && n + (uint32_t)(stream_least(B) * B) <= (uint32_t)gridDim.x
+                               ? (uint32_t)stream_least(B) : 1u;
     uint32_t pieces[4], pf[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pf[i] = pieces[i] = ceil_div_small(tiles[i], lo, rt);
+    for (int i = 0; i < 4; ++i) pf[i] = pieces[i] = max(ceil_div_small(tiles[i], lo, rt), min(tiles[i], least));
     wave_incl_scan4(pf);
     n_split = 0;
 #pragma unroll

@@ -26,19 +26,35 @@ constexpr int kGqaDevSplitMaxTiles = (1 << 17) - 1;
 // The most keys one sparse (DSA) workgroup may resolve (their row ids live in the kernel's LDS); the planner keeps to it.
 constexpr int kMlaMaxSplitKeys = 2048;
 
-// The workgroups that a paged MLA row of so many 16-key tiles is worth; a launch runs at most the sum of its rows', the
-// longest pieces as short as that many allow. A workgroup's tile loop takes time in proportion to tiles / workgroups, the
-// row's merge (a 32 KB partial a workgroup, written and read again) in proportion to the workgroups, so their sum is least
-// at sqrt(k tiles); k = 3 from sweeps of the workgroup count (graph replays, FP8 / bf16 rows, 16 heads, us: one row of
-// 4000 keys, 250 tiles: 250 workgroups 41.4 / 42.3, 63 20.5 / 19.8, 32 18.3 / 17.2, 25 18.7 / 18.2, 11 20.7 / 21.9; one of
-// 16000: 256 42.7 / 44.6, 63 24.8 / 25.8, 32 25.7 / 28.7; four of 1300-2000: 256 24.7 / 24.2, 70 18.0 / 17.4, 18 22.7 /
-// 24.0; eight of 670-1000: 256 20.4 / 18.9, 105 17.1 / 15.9, 35 19.3 / 19.3). A batch of rows of up
-// to 12 tiles, three a wave, stays whole and needs no merge (9 tiles, 32 rows: whole 14.6 / 13.6, six a row 17.5 / 15.3; 7 tiles, one row: 12.8 / 10.7, six
-// 15.9 / 13.1; at 13 tiles, one row: whole 15.2 / 14.2, eight 14.9 / 12.2).
-constexpr int32_t kStreamWholeTiles = 12;
-__host__ __device__ inline int32_t stream_pieces(int32_t tiles) {
-  return min(tiles, (int32_t)ceilf(sqrtf(3.0f * (float)tiles)));
+// The workgroups that a paged MLA row of so many 16-key tiles is worth in a batch of B rows; a launch runs at most the sum
+// of its rows', the longest pieces as short as that many allow. A workgroup's tile loop takes time in proportion to tiles /
+// workgroups, the row's merge (a 32 KB partial a workgroup, written and read again) in proportion to the workgroups, so
+// their sum is least at sqrt(k tiles); k = 3 from sweeps of the workgroup count (graph replays, FP8 / bf16 rows, 16 heads,
+// us: one row of 4000 keys, 250 tiles: 250 workgroups 41.4 / 42.3, 63 20.5 / 19.8, 32 18.3 / 17.2, 25 18.7 / 18.2, 11
+// 20.7 / 21.9; one of 16000: 256 42.7 / 44.6, 63 24.8 / 25.8, 32 25.7 / 28.7; four of 1300-2000: 256 24.7 / 24.2, 70 18.0 /
+// 17.4, 18 22.7 / 24.0; eight of 670-1000: 256 20.4 / 18.9, 105 17.1 / 15.9, 35 19.3 / 19.3).
+// Up to 16 rows take at least 8 each: the merge spreads over a row's workgroups by its 8 latent blocks, which fewer merge
+// in two turns (16 tiles, one row: 7 workgroups 15.8 / 13.1, 8 14.8 / 12.1; 16 rows: 7 17.2 / 15.3, 8 16.5 / 14.7; 32
+// rows, whose 256 workgroups then fill the chip: 7 18.2 / 16.2, 8 18.9 / 16.8).
+// Batches of more than kStreamWorthRows rows take a workgroup a CU whatever their rows are worth, at most one a tile (35
+// rows of 13 tiles are worth 245 of 256 CUs already, and a device split spends 0.1-0.2 us on the sum).
+constexpr int32_t kStreamWorthRows = 32;
+__host__ __device__ inline int32_t stream_least(int32_t B) { return B <= 16 ? 8 : 1; }
+__host__ __device__ inline int32_t stream_pieces(int32_t tiles, int32_t B) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const float root = __builtin_amdgcn_sqrtf(3.0f * (float)tiles);  // (within an ulp: one workgroup either way)
+#else
+  const float root = sqrtf(3.0f * (float)tiles);
+#endif
+  return min(tiles, max((int32_t)ceilf(root), stream_least(B)));
 }
+// A batch whose longest row has at most this many tiles stays whole, one workgroup a row and no merge: up to 8, two a
+// wave (7 tiles, one row: whole 12.9 / 10.8, seven 15.9 / 13.0); a plan from host lengths from 16 rows on up to 12 (12
+// tiles, 16 rows: whole 15.8 / 13.9, eight each 16.5 / 14.6; 32 rows: 15.8 / 14.3 and 18.9 / 16.5; but one row: 15.4 / 13.2
+// and 14.8 / 12.1, of 10 tiles 13.8 / 12.5 and 14.8 / 12.1). By the longest row, as a choice row by row in the device split
+// makes the compiler hold a buffer resource in VGPRs.
+constexpr int32_t kStreamWholeTiles = 8;
+inline int32_t stream_whole_tiles(int32_t B) { return B < 16 ? kStreamWholeTiles : 12; }
 // The MLA / DSA stream split's counter block at the start of its workspace: per (row, head group) an arrival counter
 // and a mask of merged latent blocks, then one count of finished workgroups, each in a 64-byte line of its own; zero
 // at rest. The last line holds a sticky status word: a launch that finds a counter past what a clean block allows

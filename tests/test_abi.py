@@ -231,16 +231,23 @@ def test_mla_stream_plan(lib, lens, ctas, cus):
     assert ws == 262144 + 2 * p.n_ctas * 16 * ctas * (512 + 2) * 4
 
 
-@pytest.mark.parametrize("tiles", [[1], [2], [3], [12], [13], [63], [250], [1000], [20000], [65535], [5, 400, 1],
-                                   [104] * 4, [11] * 32, [3] * 300])
+@pytest.mark.parametrize("tiles", [[1], [2], [3], [8], [9], [12], [13], [21], [22], [63], [250], [1000], [20000], [65535],
+                                   [5, 400, 1], [104] * 4, [8] * 15, [9] * 15, [12] * 16, [13] * 16, [11] * 32, [13] * 17,
+                                   [13] * 32, [13] * 33, [1] * 32 + [9], [3] * 300])
 def test_mla_plan_takes_sqrt_3_tiles_workgroups_a_row(lib, tiles):
-    """A paged row is worth ceil(sqrt(3 tiles)) workgroups (at most its tiles; a batch of rows of up to 12 tiles: one
-    each), summed over the batch and held to the launch's; the pieces are the shortest that many workgroups allow."""
+    """A paged row is worth ceil(sqrt(3 tiles)) workgroups, at least 8 in batches of up to 16 rows, at most its tiles (a
+    batch of rows of up to 8 tiles, 12 from 16 rows on: one each; of more than 32 rows: one a tile), summed over the batch
+    and held to the launch's; the pieces are the shortest that many workgroups allow."""
     import math
     tiles = tiles[:256]
+    B = len(tiles)
     rc, p = _plan(lib, _lib.KIND_MLA, [16 * t + 1 for t in tiles])
     assert rc == 0, lib.sna_last_error()
-    worth = len(tiles) if max(tiles) <= 12 else sum(min(t, math.isqrt(3 * t - 1) + 1) for t in tiles)
+    least = 8 if B <= 16 else 1
+    whole = max(tiles) <= (8 if B < 16 else 12)
+    worth = sum(tiles) if B > 32 else sum(min(t, max(least, math.isqrt(3 * t - 1) + 1)) for t in tiles)
+    if whole:
+        worth = B
     assert p.n_ctas == min(256, worth)
     _check_stream_plan(p, [16 * t for t in tiles], 256)
 

@@ -77,10 +77,13 @@ def test_mla_device_split_matches_oracle(name, over, bf16):
         assert torch.equal(scale.cpu(), scale_o), "row scales differ"
 
 
-# few rows: a row takes about sqrt(3 tiles) workgroups, one up to 12 tiles, cut on the host or on the device. (Tiles a
-# row: 1; 1, 2 and 3; 12, the longest whole row; 13; 4 and 13; a mixture; a long row.)
+# few rows: a row takes about sqrt(3 tiles) workgroups, at least 8 in up to 16 rows, one up to 8 tiles (exact plans of 16
+# rows on: 12), cut on the host or on the device. (Tiles a row: 1; 1, 2 and 3; 8, the longest whole row; 9; 12; 13; 4 and 13;
+# a mixture; a long row; 12 and 13 in 16 rows; 13 in 17; the most rows that count their worth; one past them.)
 @pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
-@pytest.mark.parametrize("lens", [[2], [17, 33, 34], [193], [194], [65, 209], [5000, 1, 60], [20001]], ids=str)
+@pytest.mark.parametrize("lens", [[2], [17, 33, 34], [129], [130], [193], [194], [65, 209], [5000, 1, 60], [20001],
+                                  [193] * 15 + [2], [194] * 15 + [2], [200] * 17, [17, 400] * 16, [17, 400] * 16 + [150]],
+                         ids=lambda v: f"{v}" if len(v) < 4 else f"{v[:2]}x{len(v)}")
 def test_mla_few_rows_match_oracle(lens, bf16):
     dev = torch.device("cuda", 0)
     case = workloads.mla_case(overrides={"B": len(lens), "fixed_lens": lens})
