@@ -5,8 +5,7 @@
 //   score of indexer_kv_score_torch_ref :254-268, indexer_topk_local_torch_ref :296-309)
 //
 // Score: one workgroup of 4 waves per (row, run of up to 4096 keys); each wave takes 16-key tiles. Bound by its key
-// loads (268 MB at about 5.2 TB/s on 16 rows of 131072 keys; with non-temporal loads, more waves or a deeper ring the
-// same). S[head, key] = Q . K^T on
+// loads (268 MB at about 5.2 TB/s on 16 rows of 131072 keys). S[head, key] = Q . K^T on
 // v_mfma_scale_f32_16x16x128_f8f6f4 (one instruction covers d = 128): lane (g4, i) feeds row i of the head tile (the
 // query split exactly into two e4m3fn parts, hi + lo / 16, of a power-of-two-scaled row, whose E8M0 A scales undo
 // the scaling) and column i, the 32 key bytes 32 g4 .. + 31 of key i, loaded straight from HBM into a register ring.
@@ -50,27 +49,35 @@ __device__ __forceinline__ f32x4_t mfma_16x16x128_fp8_sa(const uint32_t (&a)[8],
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, scale_a, 0, 127);
 }
 
-// Keys per workgroup: a multiple of kScoreStep (PD steps of the four waves' 64 keys), at most kScoreKeys. The host picks
-// the number that gives the launch about kScoreBlocks workgroups, two a CU, in one round: 16 rows of 131072 keys (64
-// heads), store, scores and top-k 77.8 -> 74.5 us against 2048 keys a workgroup in two rounds (768 workgroups 79.7, 1024
-// 80.7, 1536 85.5 with the non-temporal loads), one row of 131072 or four of 32768 31.5 -> 26.5.
-constexpr int kScoreKeys = 4096, kScoreStep = 256, kScoreBlocks = 512;
+// Keys per workgroup: a multiple of kScoreStep (whole turns of the ring), from kScoreMinKeys (two turns of four tiles a
+// wave; one row of 500 keys takes 5.7 us as one run, of 131072 6.1 as 256, so a run is mostly its prologue) to kScoreKeys
+// (LDS), the least with which the launch has at most kScoreBlocks workgroups, two a CU: 128 heads' registers hold no more,
+// and with 64 heads one round of long runs beat two of 2048 keys (16 rows of 131072 46.1 -> 44.5 us, of 20000 12.3 -> 10.4;
+// 513 workgroups instead of 512 cost three rows of 131072 15.9 instead of 13.0). With 16 and 32 heads, which hold more, 16
+// uniform rows of 131072 take 44.4 / 44.9 us so and 43.6 with three a CU, 42.5 / 43.0 with four, but ragged rows lose by it
+// (16 of 1000 to 131072, in any order: 34.3-35.2, 36.2-37.7 and 36.0-37.4).
+// Workgroups go run by run, then row by row, so that with ragged rows those that hold no live key come last (16 rows of
+// 4000-8000 of a table of 65536, 64 heads: 21.4 -> 12.0 us; a row's runs in turn left CUs idle by the rows' order).
+constexpr int kScoreKeys = 4096, kScoreStep = 256, kScoreMinKeys = 512, kScoreBlocks = 512;
+constexpr int kScoreGridY = 32768;  // runs of the grid's second dimension (the third holds the others)
 
 template <int HT>  // head tiles of 16
 __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
   // PD: key tiles each wave has in flight ahead of the one it scores (fewer with 128 heads, whose query operands
   // take 128 VGPRs)
   constexpr int D = 128, PD = HT >= 8 ? 2 : 4;
-  static_assert(kScoreStep % (64 * PD) == 0 && kScoreKeys % kScoreStep == 0, "whole turns of the ring");
+  static_assert(kScoreStep % (64 * PD) == 0 && kScoreMinKeys % kScoreStep == 0 && kScoreKeys % kScoreStep == 0,
+                "whole turns of the ring");
   __shared__ uint32_t sm_q[HT][2][8][64];  // [head tile][hi, lo][dword][lane]: the MFMA A operand of each lane
   __shared__ int32_t sm_ex[HT][64];         // floor(log2 amax) of the head lane (li) feeds, per head tile
   __shared__ int32_t sm_row[kScoreKeys];    // the keys' byte offsets in the cache / 16 (under 2^31), -1: dead
   __shared__ __align__(16) uint16_t sm_out[kScoreKeys];  // the workgroup's bf16 scores
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int32_t b = blockIdx.y;
-  const int32_t e_blk = (int32_t)blockIdx.x * a.keys_wg;
-  if (e_blk >= a.width) return;
+  const int32_t b = blockIdx.x;
+  const int64_t e_first = (int64_t)(blockIdx.y + gridDim.y * blockIdx.z) * a.keys_wg;
+  if (e_first >= a.width) return;
+  const int32_t e_blk = (int32_t)e_first;
   const int32_t limit = a.limits[b];
   const int32_t* trow = a.table + (int64_t)b * a.table_stride;
 
@@ -86,6 +93,14 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
       for (int c = 0; c < 4; ++c) qraw[j][c] = ld16(qp + 8 * c);
     }
   }
+
+  // weights of heads 16 ht + 4 g4 + r (the rows this lane's results hold), times d^-0.5: w relu(s d^-0.5) =
+  // (w d^-0.5) relu(s) as d^-0.5 > 0
+  float wl[HT][4];
+#pragma unroll
+  for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wl[ht][r] = a.w[(int64_t)b * a.H + 16 * ht + 4 * g4 + r] * a.scale;
 
   // The keys' rows: thread t resolves keys e_blk + t, + 256, ..., eight lookups in flight. (col, off) = divmod(e, P),
   // stepped by 256 keys: one division for the first, then (col, off) += divmod(256, P) with at most one carry.
@@ -112,9 +127,34 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     }
   }
 
+  __syncthreads();
+  // Key tiles in flight: tile t's (keys 64 t + 16 wave + li) 32 bytes of this lane land in ring[t % PD], its row offset in
+  // kof[t % PD]; knx[t % PD] is the offset of the tile loaded next there, read from LDS a turn ahead, so no load's address
+  // waits for LDS. The first tiles load before the queries are split. Every lane loads (a dead key reads row 0 of the cache,
+  // in bounds, and its score is replaced), so no branch or store sits between a load and its use and the waits count only
+  // the ring's own loads. (Instructions of 64 contiguous bytes a key measured the same, and sum the dims in another order.)
+  // Plain loads: with the non-temporal hint 16 rows of 65536 keys, half of them in the Infinity Cache, took 49.5 us instead
+  // of 45.7 (16 of 131072 the same). These two orders took one row of 2048 keys from 6.4 to 5.9 us (64 heads; 16 heads 5.9
+  // to 5.2); a ring of 8 measured slower (16 heads 6.0).
+  uint32_t ring[PD][8];
+  int32_t kof[PD], knx[PD];
+  const int32_t* my_row = &sm_row[16 * wave + li];
+  auto fetch = [&](int32_t t_after, int u) {
+    kof[u] = knx[u];
+    knx[u] = my_row[64 * t_after];
+    const uint8_t* kp = a.keys + ((int64_t)max(kof[u], 0) << 4) + 32 * g4;
+    const uint4 x0 = ld16(kp), x1 = ld16(kp + 16);
+    ring[u][0] = x0.x, ring[u][1] = x0.y, ring[u][2] = x0.z, ring[u][3] = x0.w;
+    ring[u][4] = x1.x, ring[u][5] = x1.y, ring[u][6] = x1.z, ring[u][7] = x1.w;
+  };
+#pragma unroll
+  for (int u = 0; u < PD; ++u) knx[u] = my_row[64 * u];
+#pragma unroll
+  for (int u = 0; u < PD; ++u) fetch(min(u + PD, a.keys_wg / 64 - 1), u);  // (no tile past those resolved above)
+
   // The query operand of head tile ht: lane (g4, i) supplies head 16 ht + i, dims 32 g4 .. + 31, as two exact e4m3fn
-  // parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over the head's 128 dims); the E8M0 A scales are 127 - log2 sc for hi and 4 less for lo. Wave w splits head tiles w,
-  // w + 4, ... into LDS.
+  // parts of the row scaled by sc = 2^(7 - floor(log2 amax)) (amax over the head's 128 dims); the E8M0 A scales are 127 -
+  // log2 sc for hi and 4 less for lo. Wave w splits head tiles w, w + 4, ... into LDS.
 #pragma unroll
   for (int j = 0; j < QT; ++j) {
     const int ht = wave + 4 * j;
@@ -146,32 +186,7 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     }
     sm_ex[ht][lane] = ex;
   }
-  // weights of heads 16 ht + 4 g4 + r (the rows this lane's results hold), times d^-0.5: w relu(s d^-0.5) =
-  // (w d^-0.5) relu(s) as d^-0.5 > 0
-  float wl[HT][4];
-#pragma unroll
-  for (int ht = 0; ht < HT; ++ht)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) wl[ht][r] = a.w[(int64_t)b * a.H + 16 * ht + 4 * g4 + r] * a.scale;
-
   __syncthreads();
-  // Key tiles in flight: tile t's (keys 64 t + 16 wave + li) 32 bytes of this lane land in ring[t % PD], its row offset in
-  // kof[t % PD]. Every lane loads (a dead key reads row 0 of the cache, in bounds, and its score is replaced), so no
-  // branch or store sits between a load and its use and the waits count only the ring's own loads. (Instructions of 64
-  // contiguous bytes a key measured the same, and sum the dims in another order.) Plain loads: with the non-temporal hint 16 rows of 65536 keys, half of them in
-  // the Infinity Cache, took 49.5 us instead of 45.7 (16 of 131072 the same).
-  const int32_t tiles = a.keys_wg / 64;
-  uint32_t ring[PD][8];
-  int32_t kof[PD];
-  auto fetch = [&](int32_t t, int u) {
-    kof[u] = sm_row[64 * t + 16 * wave + li];
-    const uint8_t* kp = a.keys + ((int64_t)max(kof[u], 0) << 4) + 32 * g4;
-    const uint4 x0 = ld16(kp), x1 = ld16(kp + 16);
-    ring[u][0] = x0.x, ring[u][1] = x0.y, ring[u][2] = x0.z, ring[u][3] = x0.w;
-    ring[u][4] = x1.x, ring[u][5] = x1.y, ring[u][6] = x1.z, ring[u][7] = x1.w;
-  };
-#pragma unroll
-  for (int u = 0; u < PD; ++u) fetch(u, u);
   uint32_t qhi[HT][8], qlo[HT][8];
   int32_t sc_hi[HT], sc_lo[HT];
 #pragma unroll
@@ -183,8 +198,10 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
     sc_lo[ht] = 127 + ex - 7 - 4;
   }
 
-  // scores of the workgroup's keys, written out coalesced at the end
-  for (int32_t t0 = 0; t0 < tiles; t0 += PD) {
+  // scores of the workgroup's keys, written out coalesced at the end: only tiles that hold a key below the row's limit, in
+  // whole turns of the ring; past them every key is dead
+  const int32_t live = (min(max(min(limit, a.width) - e_blk, 0), a.keys_wg) + 64 * PD - 1) / (64 * PD) * PD;
+  for (int32_t t0 = 0; t0 < live; t0 += PD) {
 #pragma unroll
     for (int u = 0; u < PD; ++u) {
       float sum = 0.0f;
@@ -197,13 +214,14 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a) {
         for (int r = 0; r < 4; ++r)  // relu as an integer max: a negative float's bits are a negative integer
           sum = fmaf(wl[ht][r], __int_as_float(max(__float_as_int(s[r]), 0)), sum);
       }
-      const bool live = kof[u] >= 0;
-      fetch(min(t0 + u + PD, tiles - 1), u);  // (past the last tile: it again, not used)
+      const bool key_live = kof[u] >= 0;
+      fetch(min(t0 + u + 2 * PD, live - 1), u);  // (past the last tile: it again, not used)
       sum = sum_across_groups(sum);  // every lane of key li holds the key's sum
       sm_out[64 * (t0 + u) + 16 * wave + li] =
-          (uint16_t)f32_to_bf16_bits(live ? fminf(sum, kIndexMaskBound) : -kIndexMaskBound);
+          (uint16_t)f32_to_bf16_bits(key_live ? fminf(sum, kIndexMaskBound) : -kIndexMaskBound);
     }
   }
+  for (int32_t i = 64 * live + tid; i < a.keys_wg; i += 256) sm_out[i] = (uint16_t)f32_to_bf16_bits(-kIndexMaskBound);
   __syncthreads();
   uint16_t* orow = a.out + (int64_t)b * a.out_stride + e_blk;
   const int32_t n = min(a.keys_wg, a.width - e_blk);
@@ -537,10 +555,13 @@ int sna_indexer_scores(const void* q, const float* w, const uint8_t* keys, const
   a.P = page_size;
   a.num_blocks = num_blocks;
   a.scale = 1.0f / sqrtf((float)head_dim);
-  const int64_t per = ((int64_t)B * width + kScoreBlocks - 1) / kScoreBlocks;
-  a.keys_wg = (int32_t)std::min<int64_t>(kScoreKeys, std::max<int64_t>(2 * kScoreStep,
-                                                                      (per + kScoreStep - 1) / kScoreStep * kScoreStep));
-  const dim3 grid((unsigned)((width + a.keys_wg - 1) / a.keys_wg), (unsigned)B);
+  a.keys_wg = kScoreMinKeys;
+  auto runs_of = [&](int32_t keys) -> int64_t { return ((int64_t)width + keys - 1) / keys; };
+  while (a.keys_wg < kScoreKeys && runs_of(a.keys_wg) > 1 && B * runs_of(a.keys_wg) > kScoreBlocks)
+    a.keys_wg += kScoreStep;
+  const int64_t runs = runs_of(a.keys_wg);
+  const dim3 grid((unsigned)B, (unsigned)std::min<int64_t>(runs, kScoreGridY),
+                  (unsigned)((runs + kScoreGridY - 1) / kScoreGridY));
   const hipStream_t s = (hipStream_t)stream;
   switch (num_heads / 16) {
     case 1: hipLaunchKernelGGL((indexer_score_kernel<1>), grid, dim3(256), 0, s, a); break;

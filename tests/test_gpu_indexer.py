@@ -68,6 +68,40 @@ def test_indexer_scores_match_oracle(name, seed, H, P, limits, width):
     assert bool((err <= bound).all()), f"{name}: max err {float(err.max())}"
 
 
+# the workgroups' run lengths: the least multiple of 256 keys with B * ceil(width / keys) <= 512, in 512 .. 4096 (a row's own)
+LONG = [("512-keys", 64, 64, 16, 4096), ("768-keys", 64, 64, 48, 5900), ("2048-keys-h16", 16, 64, 64, 16383),
+        ("2304-keys", 64, 64, 48, 17801), ("3328-keys-h32", 32, 64, 16, 26001), ("4096-keys-two-rounds", 64, 61, 64, 40003),
+        ("4096-keys-h128", 128, 64, 80, 32768), ("more-rows-than-workgroups", 16, 700, 16, 530)]
+
+
+@pytest.mark.parametrize("name,H,B,P,width", LONG, ids=[c[0] for c in LONG])
+def test_indexer_scores_run_lengths(name, H, B, P, width):
+    """Batches whose workgroups take long runs of keys: every row's scores are the bits of that row scored alone (short
+    runs), and a few rows' match the oracle; rows end inside runs, before them and past the width, pages are invalid."""
+    announce(f"indexer score runs {name}: B={B} H={H} P={P} width={width}")
+    g = torch.Generator().manual_seed(width)
+    nb, pages = 200, -(-width // P)
+    table = torch.randint(1, nb, (B, pages), generator=g, dtype=torch.int32)
+    table[torch.rand(B, pages, generator=g) < 0.01] = -1
+    cache = oix.pack_index_keys(torch.randn(nb * P, 128, generator=g).to(torch.bfloat16) * 1.5).reshape(nb, P, 128)
+    q = torch.randn(B, H, 128, generator=g).to(torch.bfloat16)
+    w = torch.randn(B, H, generator=g) * H ** -0.5
+    lim = torch.randint(0, width + 50, (B,), generator=g, dtype=torch.int32)
+    lim[0], lim[1], lim[2], lim[-1] = width, 0, 4097, width - 1
+    d = [t.to(DEV) for t in (q, w, cache, table, lim)]
+    got = ops.indexer_scores(*d, width)
+    for b in range(0, B, max(1, B // 64)):
+        one = ops.indexer_scores(d[0][b:b + 1], d[1][b:b + 1], d[2], d[3][b:b + 1], d[4][b:b + 1], width)
+        assert torch.equal(one[0], got[b]), f"row {b}"
+    rows = [0, 2, B - 1]
+    want = oix.indexer_scores(q[rows], w[rows], cache, table[rows], lim[rows], width).float()
+    mine = got.cpu()[rows].float()
+    dead = want <= -5e29
+    assert torch.equal(mine[dead], want[dead]), "dead keys must score -1e30"
+    bound = want[~dead].abs() * 2.0 ** -7 + 2e-4  # one bf16 rounding (and fp32 sum order under cancellation)
+    assert bool(((mine[~dead] - want[~dead]).abs() <= bound).all())
+
+
 def _deterministic_topk(row: torch.Tensor, k: int) -> set:
     """The selection with ties taken at the lowest positions (sort by value desc, then position), dead keys as -1."""
     r = row.float().tolist()
