@@ -232,13 +232,20 @@ __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32
   return found;
 }
 
-template <int D, int ESZ, bool SPLIT>
+// kOneTile and kHalfTile: the launch's tables name at most one tile of keys, or 32 of them (prompts of up to 64 or 32 tokens
+// with no prior), so the loop's next tile, whose products it computes whether there is one or not, and the tile's second
+// sub-tile are left out (32 / 8 heads of 128, FP8 / bf16, us: 16 tokens 8.2 / 7.6 through the loop, 6.9 / 6.2 so; 60 tokens 9.0 /
+// 8.4 and 8.7 / 8.0; as runtime branches of one kernel 7.8 / 7.4 and 9.1 / 9.0).
+enum PrefillMode { kWhole, kSplit, kOneTile, kHalfTile };
+template <int D, int ESZ, PrefillMode MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_gqa_kernel(PrefillArgs a) {
   using Geo = PrefillGeo<D, ESZ>;
-  constexpr int ROWB = Geo::ROWB, CH = Geo::CH, HALF = Geo::HALF, SLOT = Geo::SLOT, TK = Geo::TK, NSUB = Geo::NSUB;
+  constexpr int ROWB = Geo::ROWB, CH = Geo::CH, HALF = Geo::HALF, SLOT = Geo::SLOT;
+  constexpr bool ONE = MODE == kOneTile || MODE == kHalfTile;
+  constexpr int TK = MODE == kHalfTile ? Geo::TK / 2 : Geo::TK, NSUB = TK / 32;
   constexpr int MW = Geo::MW, RPD = Geo::RPD;
-  constexpr bool FP8 = ESZ == 1;
+  constexpr bool FP8 = ESZ == 1, SPLIT = MODE == kSplit;
   constexpr int NS = FP8 ? D / 64 : D / 16;  // QK steps
   constexpr int NC = D / 32;                 // PV dim tiles
   typedef __attribute__((address_space(3))) void lds_void;
@@ -507,7 +514,8 @@ void prefill_gqa_kernel(PrefillArgs a) {
   __builtin_amdgcn_s_waitcnt(0x0f70);
 
   const int32_t t_first = blk.t0 + (SPLIT ? split * split_tiles : 0);
-  const int32_t t_end = SPLIT ? min(blk.t1, t_first + split_tiles) : blk.t1;
+  // (ONE: a length past the table has only invalid keys in its other tiles)
+  const int32_t t_end = SPLIT ? min(blk.t1, t_first + split_tiles) : ONE ? min(blk.t1, t_first + 1) : blk.t1;
   const int32_t chunk_tiles = (Geo::PAGES - 1) * a.P / TK;  // (a chunk may start mid-page: PAGES - 1 whole pages)
   for (int32_t c0 = t_first; c0 < t_end; c0 += chunk_tiles) {
     const int32_t c1 = min(c0 + chunk_tiles, t_end);
@@ -529,8 +537,10 @@ void prefill_gqa_kernel(PrefillArgs a) {
     int32_t pg = page_of(c0);
     uint32_t ok_cur = pages_ok(pg), ok_next;
     int64_t off = group_off(c0, pg);
-    load(kg + off, ring);
-    load(vg + off, ring + HALF);
+    if (TK / 16 == 4 || wave < TK / 16) {
+      load(kg + off, ring);
+      load(vg + off, ring + HALF);
+    }
     pg = page_of(min(c0 + 1, c1 - 1));
     ok_next = pages_ok(pg);
     off = group_off(min(c0 + 1, c1 - 1), pg);  // of tile i + 1
@@ -541,18 +551,8 @@ void prefill_gqa_kernel(PrefillArgs a) {
     f32x16_t sa[NSUB], sb[NSUB];
     qk(&sm_ring[0], sa);
     exponents(sa);
-    auto step = [&](int32_t i, auto parity, f32x16_t (&cur)[NSUB], f32x16_t (&next)[NSUB]) {
-      constexpr int P = decltype(parity)::value;  // i % 2
-      wait_vmcnt<0>();  // this wave's K of tile i + 1 and V of tile i have landed
-      // every wave's have; every wave is done with K of tile i and V of tile i - 1 (their slots are free)
-      __syncthreads();
-      if (i + 1 < n) load(vg + off, ring + (1 - P) * SLOT + HALF);
-      const uint32_t ok2 = pages_ok(pg);
-      if (i + 2 < n) {
-        off = group_off(c0 + i + 2, pg);
-        load(kg + off, ring + P * SLOT);
-        pg = page_of(min(c0 + i + 3, c1 - 1));
-      }
+    // tile i (in ring slot P) up to its exponents under the reference maximum: V cleaned, scores masked
+    auto settle = [&](int32_t i, int P, f32x16_t (&cur)[NSUB]) {
       const int32_t k0 = TK * (c0 + i);
       const bool valid = ok_cur == (1u << (TK / 16)) - 1;
       if (!valid || k0 + TK > hi) {
@@ -568,20 +568,40 @@ void prefill_gqa_kernel(PrefillArgs a) {
       // a tile that is not full (a key invalid or not visible to every row of the block) masks its scores
       if (!valid || k0 + TK - 1 > pos0 || (a.window != 0 && k0 <= hi - 1 - a.window)) mask(k0, ok_cur, cur);
       if (any_unset || __any(mx > kPrefillRescaleSlack)) move_reference(cur);
-      qk(&sm_ring[(1 - P) * SLOT], next);  // (past the last tile: whatever the slot holds, not used)
-      probabilities(cur);
-      pv(&sm_ring[P * SLOT]);
-      exponents(next);
-      // (a use here, so the compiler does not move the next tile's products past the loop's exit test)
-      asm volatile("" : "+v"(mx), "+v"(next[0]), "+v"(next[1]));
-      ok_cur = ok_next;
-      ok_next = ok2;
     };
-    for (int32_t i = 0;;) {
-      step(i, std::integral_constant<int, 0>{}, sa, sb);
-      if (++i >= n) break;
-      step(i, std::integral_constant<int, 1>{}, sb, sa);
-      if (++i >= n) break;
+    if constexpr (ONE) {
+      settle(0, 0, sa);
+      probabilities(sa);
+      pv(&sm_ring[0]);
+    } else {
+      auto step = [&](int32_t i, auto parity, f32x16_t (&cur)[NSUB], f32x16_t (&next)[NSUB]) {
+        constexpr int P = decltype(parity)::value;  // i % 2
+        wait_vmcnt<0>();  // this wave's K of tile i + 1 and V of tile i have landed
+        // every wave's have; every wave is done with K of tile i and V of tile i - 1 (their slots are free)
+        __syncthreads();
+        if (i + 1 < n) load(vg + off, ring + (1 - P) * SLOT + HALF);
+        const uint32_t ok2 = pages_ok(pg);
+        if (i + 2 < n) {
+          off = group_off(c0 + i + 2, pg);
+          load(kg + off, ring + P * SLOT);
+          pg = page_of(min(c0 + i + 3, c1 - 1));
+        }
+        settle(i, P, cur);
+        qk(&sm_ring[(1 - P) * SLOT], next);  // (past the last tile: whatever the slot holds, not used)
+        probabilities(cur);
+        pv(&sm_ring[P * SLOT]);
+        exponents(next);
+        // (a use here, so the compiler does not move the next tile's products past the loop's exit test)
+        asm volatile("" : "+v"(mx), "+v"(next[0]), "+v"(next[1]));
+        ok_cur = ok_next;
+        ok_next = ok2;
+      };
+      for (int32_t i = 0;;) {
+        step(i, std::integral_constant<int, 0>{}, sa, sb);
+        if (++i >= n) break;
+        step(i, std::integral_constant<int, 1>{}, sb, sa);
+        if (++i >= n) break;
+      }
     }
   }
 
@@ -704,11 +724,15 @@ int64_t split_workspace_bytes(int32_t slots, int32_t R, int32_t max_q_len, int32
 template <int D, int ESZ>
 void launch_prefill(const PrefillArgs& a, hipStream_t s) {
   if (a.slots > 0) {
-    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, true>), dim3(a.slots), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, kSplit>), dim3(a.slots), dim3(256), 0, s, a);
     hipLaunchKernelGGL((prefill_combine_kernel<D>), dim3(kPrefillRows * D / 1024 * a.qblocks, a.R, a.G),
                        dim3(256), 0, s, a, ESZ == 1);
+  } else if ((int64_t)a.table_width * a.P <= kPrefillTile / 2) {
+    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, kHalfTile>), dim3(a.qblocks, a.R, a.G), dim3(256), 0, s, a);
+  } else if ((int64_t)a.table_width * a.P <= kPrefillTile) {
+    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, kOneTile>), dim3(a.qblocks, a.R, a.G), dim3(256), 0, s, a);
   } else {
-    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, false>), dim3(a.qblocks, a.R, a.G), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((prefill_gqa_kernel<D, ESZ, kWhole>), dim3(a.qblocks, a.R, a.G), dim3(256), 0, s, a);
   }
 }
 

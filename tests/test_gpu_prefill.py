@@ -145,15 +145,58 @@ def test_prefill_split_edges(name, seed, cfg, window, sinks):
                                 v_scale=vsd, sinks=skd, window=window)
     torch.cuda.synchronize()
     assert_close_attn(out.cpu(), want, name)
-    whole = torch.empty_like(out)
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    rc = lib.sna_prefill_attention(ptr(qd), ptr(kc), ptr(vc), ptr(ksd), ptr(vsd), ptr(td), td.stride(0), width, ptr(sd),
-                                   ptr(pd), R, longest, ptr(skd), d ** -0.5, window, ptr(whole), H, G, d, P,
-                                   kc.shape[0], _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_FP8_E4M3FN,
-                                   torch.cuda.current_stream().cuda_stream)
-    assert rc == 0, _lib.last_error()
+    whole = _unsplit(qd, kc, vc, ksd, vsd, td, sd, pd, longest, d ** -0.5, window, skd)
     torch.cuda.synchronize()
     assert_close_attn(whole.cpu(), want, f"{name} unsplit")
+
+
+def _unsplit(q, kc, vc, ks, vs, table, q_start, priors, longest, scale, window=0, sinks=None):
+    """sna_prefill_attention: the entry without a workspace, which never splits. Device tensors."""
+    lib = _lib.load()
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    out = torch.empty_like(q)
+    rc = lib.sna_prefill_attention(ptr(q), ptr(kc), ptr(vc), ptr(ks), ptr(vs), ptr(table), table.stride(0), table.shape[1],
+                                   ptr(q_start), ptr(priors), priors.numel(), longest, ptr(sinks), scale, window, ptr(out),
+                                   q.shape[1], kc.shape[1], q.shape[2], kc.shape[2], kc.shape[0],
+                                   _lib.DTYPE_BF16 if ks is None else _lib.DTYPE_FP8_E4M3FN,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    return out
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("P", [16, 48, 64])
+def test_prefill_one_tile(P, d, bf16):
+    """Prompts whose tables name at most 64 keys (a kernel of their own): within the attention bar of the oracle, and the
+    bits of the general kernel over a wider table, with NaN in every slot no query may see and pages of -1 past the prompt."""
+    announce(f"prefill one tile P={P} d={d} bf16={bf16}")
+    H, G = 8, 2
+    for lens, window in (((1,), 0), ((16, 3), 0), ((17, 32), 5), ((33,), 0), ((48, 1, 20), 0), ((49, 63), 40), ((64,), 0)):
+        if max(lens) > 64 // P * P:
+            continue
+        n, R = max(lens), len(lens)
+        q, kc, vc, ks, vs, table, q_start, priors = _case(51 + n, H=H, G=G, d=d, P=P, priors=(0,) * R, lens=lens, bf16=bf16)
+        used = torch.zeros(kc.shape[0] * P, dtype=torch.bool)
+        for r, m in enumerate(lens):
+            at = torch.arange(m)
+            used[table[r, at // P].long() * P + at % P] = True
+        dead = (~used).reshape(kc.shape[0], 1, P, 1).to(DEV)
+        kh, vh = (kc.cpu(), vc.cpu()) if bf16 else (kc.cpu().view(torch.uint8), vc.cpu().view(torch.uint8))
+        for cache in (kc, vc):
+            cache.view(torch.int16 if bf16 else torch.uint8).masked_fill_(dead, 0x7FC0 if bf16 else 0x7F)
+        want = oatt.segmented_prefill(q, kh, vh, table, q_start, priors, sm_scale=d ** -0.5, k_scale=ks, v_scale=vs,
+                                      sinks=None, window=window)
+        kd, vd = (None, None) if bf16 else (ks.to(DEV), vs.to(DEV))
+        qd, sd, pd = q.to(DEV), q_start.to(DEV), priors.to(DEV)
+        narrow = table[:, :-(-n // P)].contiguous().to(DEV)
+        assert narrow.shape[1] * P <= 64
+        out = ops.prefill_attention(qd, kc, vc, narrow, sd, pd, max_q_len=n, sm_scale=d ** -0.5, k_scale=kd, v_scale=vd,
+                                    window=window)
+        assert_close_attn(out.cpu(), want, f"{lens}")
+        wide = torch.full((R, 8), -1, dtype=torch.int32)
+        wide[:, :min(8, table.shape[1])] = table[:, :8]
+        assert torch.equal(out, _unsplit(qd, kc, vc, kd, vd, wide.to(DEV), sd, pd, n, d ** -0.5, window)), lens
 
 
 @pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
