@@ -52,6 +52,20 @@ def _case(seed, H, G, d, P, priors, lens, spare_pages=5, bf16=False):
     return q, kc, vc, ks, vs, table, q_start, torch.tensor(priors, dtype=torch.int32)
 
 
+def _unsplit(q, kc, vc, ks, vs, table, q_start, priors, longest, scale, window=0, sinks=None):
+    """sna_prefill_attention: the entry without a workspace, which never splits. Device tensors."""
+    lib = _lib.load()
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    out = torch.empty_like(q)
+    rc = lib.sna_prefill_attention(ptr(q), ptr(kc), ptr(vc), ptr(ks), ptr(vs), ptr(table), table.stride(0), table.shape[1],
+                                   ptr(q_start), ptr(priors), priors.numel(), longest, ptr(sinks), scale, window, ptr(out),
+                                   q.shape[1], kc.shape[1], q.shape[2], kc.shape[2], kc.shape[0],
+                                   _lib.DTYPE_BF16 if ks is None else _lib.DTYPE_FP8_E4M3FN,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    return out
+
+
 CASES = [
     ("qwen3-8b-chunks", 1, dict(H=32, G=8, d=128, P=16, priors=(0, 100, 1000), lens=(64, 200, 37)), 0, False),
     ("gpt-oss-swa-sinks", 2, dict(H=8, G=1, d=64, P=16, priors=(300, 0), lens=(150, 129)), 128, True),
@@ -72,21 +86,26 @@ CASES = [
 
 @pytest.mark.parametrize("name,seed,cfg,window,sinks", CASES, ids=[c[0] for c in CASES])
 def test_prefill_attention_matches_oracle(name, seed, cfg, window, sinks):
+    """Each case as the package calls it (long priors split their keys) and through the entry that never splits, whose
+    workgroups then walk every key: more than the block-table entries staged at a time (2047 pages) in the long cases."""
     announce(f"prefill {name}: {cfg} window={window} sinks={sinks}")
     q, kc, vc, ks, vs, table, q_start, priors = _case(seed, **cfg)
     H, d = cfg["H"], cfg["d"]
     sk = torch.randn(H, generator=torch.Generator().manual_seed(seed + 50)) if sinks else None
     scale = d ** -0.5
     bf16 = cfg.get("bf16", False)
-    out = ops.prefill_attention(q.to(DEV), kc, vc, table.to(DEV), q_start.to(DEV), priors.to(DEV),
-                                max_q_len=max(cfg["lens"]) + 7, sm_scale=scale,
-                                k_scale=None if bf16 else ks.to(DEV), v_scale=None if bf16 else vs.to(DEV),
-                                sinks=None if sk is None else sk.to(DEV), window=window)
+    longest = max(cfg["lens"]) + 7
+    kd, vd = (None, None) if bf16 else (ks.to(DEV), vs.to(DEV))
+    skd = None if sk is None else sk.to(DEV)
+    args = (q.to(DEV), kc, vc, table.to(DEV), q_start.to(DEV), priors.to(DEV))
+    out = ops.prefill_attention(*args, max_q_len=longest, sm_scale=scale, k_scale=kd, v_scale=vd, sinks=skd, window=window)
+    whole = _unsplit(*args[:3], kd, vd, *args[3:], longest, scale, window, skd)
     torch.cuda.synchronize()
     kh, vh = (kc.cpu(), vc.cpu()) if bf16 else (kc.cpu().view(torch.uint8), vc.cpu().view(torch.uint8))
     want = oatt.segmented_prefill(q, kh, vh, table, q_start, priors, sm_scale=scale, k_scale=ks, v_scale=vs, sinks=sk,
                                   window=window)
     assert_close_attn(out.cpu(), want, name)
+    assert_close_attn(whole.cpu(), want, f"{name} unsplit")
 
 
 def _random_shape(seed: int):
@@ -111,25 +130,36 @@ def test_prefill_random_shape(seed):
     test_prefill_attention_matches_oracle(f"random-{seed}", seed, cfg, window, sinks)
 
 
-# the split's edges: one tile past the least table that splits (and too few to pay), a block's keys cut into many splits,
-# splits under a window, a group that does not divide a block's rows, chunks of unequal length (query blocks that do not
-# exist), as many blocks as a split launch takes
+# the split's edges: one tile past the least table that splits, a block's keys cut into many splits, splits under a window, a
+# group that does not divide a block's rows, chunks of unequal length (query blocks that do not exist), as many blocks as a
+# split launch takes, a wide table over keys too few to pay (the device drops the split)
 SPLIT_CASES = [
-    ("seventeen-tiles", 21, dict(H=8, G=2, d=128, P=16, priors=(1025, 0), lens=(60, 5)), 0, False),
-    ("forty-tiles", 27, dict(H=8, G=2, d=128, P=16, priors=(2500, 1030), lens=(60, 5)), 0, False),
-    ("many-splits-d64", 22, dict(H=4, G=1, d=64, P=16, priors=(20000, 3), lens=(9, 70)), 0, True),
-    ("window-splits-bf16", 23, dict(H=8, G=1, d=128, P=64, priors=(9000, 700), lens=(40, 30), bf16=True), 3000, True),
-    ("group3-splits", 24, dict(H=6, G=2, d=64, P=48, priors=(2500,), lens=(43,), bf16=True), 0, False),
-    ("most-blocks", 25, dict(H=16, G=8, d=64, P=16, priors=(1600, 0), lens=(33, 1024)), 0, False),
+    ("seventeen-tiles", 21, dict(H=8, G=2, d=128, P=16, priors=(1025, 0), lens=(60, 5)), 0, False, 3),
+    ("forty-tiles", 27, dict(H=8, G=2, d=128, P=16, priors=(2500, 1030), lens=(60, 5)), 0, False, 5),
+    ("many-splits-d64", 22, dict(H=4, G=1, d=64, P=16, priors=(20000, 3), lens=(9, 70)), 0, True, 40),
+    ("window-splits-bf16", 23, dict(H=8, G=1, d=128, P=64, priors=(9000, 700), lens=(40, 30), bf16=True), 3000, True, 6),
+    ("group3-splits", 24, dict(H=6, G=2, d=64, P=48, priors=(2500,), lens=(43,), bf16=True), 0, False, 5),
+    ("most-blocks", 25, dict(H=16, G=8, d=64, P=16, priors=(1600, 0), lens=(33, 1024)), 0, False, 4),
+    ("dropped", 28, dict(H=8, G=2, d=128, P=16, priors=(600, 30), lens=(60, 5)), 0, True, 1),
 ]
 
 
-@pytest.mark.parametrize("name,seed,cfg,window,sinks", SPLIT_CASES, ids=[c[0] for c in SPLIT_CASES])
-def test_prefill_split_edges(name, seed, cfg, window, sinks):
-    """Launches that split the keys, at the sizes where a split can go wrong; then the same call through the entry that
-    takes no workspace (which never splits): both within the attention bar of the oracle."""
+def _splits_run(ws, slots, R, blocks, G, d):
+    """The split count of every (KV head, request, query block) a split launch left in its workspace (blocks a request does
+    not have keep what the workspace held)."""
+    at = slots * 128 * (d + 2) * 4
+    return ws[at:at + 8 * G * R * blocks].view(torch.int32).reshape(G, R, blocks, 2)[..., 1].cpu()
+
+
+@pytest.mark.parametrize("name,seed,cfg,window,sinks,most", SPLIT_CASES, ids=[c[0] for c in SPLIT_CASES])
+def test_prefill_split_edges(name, seed, cfg, window, sinks, most):
+    """Launches that may split the keys, at the sizes where a split can go wrong; then the same call through the entry that
+    takes no workspace (which never splits): both within the attention bar of the oracle. most: at least so many splits of
+    a query block ran, or (1) the device dropped the split."""
     announce(f"prefill split {name}: {cfg} window={window} sinks={sinks}")
     q, kc, vc, ks, vs, table, q_start, priors = _case(seed, **cfg)
+    if most == 1:
+        table = torch.cat([table, torch.full((len(table), 200), -1, dtype=torch.int32)], dim=1)
     H, G, d, P, bf16 = cfg["H"], cfg["G"], cfg["d"], cfg["P"], cfg.get("bf16", False)
     R, longest, width = len(cfg["lens"]), max(cfg["lens"]), table.shape[1]
     sk = torch.randn(H, generator=torch.Generator().manual_seed(seed + 50)) if sinks else None
@@ -141,27 +171,29 @@ def test_prefill_split_edges(name, seed, cfg, window, sinks):
     kh, vh = (kc.cpu(), vc.cpu()) if bf16 else (kc.cpu().view(torch.uint8), vc.cpu().view(torch.uint8))
     want = oatt.segmented_prefill(q, kh, vh, table, q_start, priors, sm_scale=d ** -0.5, k_scale=ks, v_scale=vs,
                                   sinks=sk, window=window)
-    out = ops.prefill_attention(qd, kc, vc, td, sd, pd, max_q_len=longest, sm_scale=d ** -0.5, k_scale=ksd,
-                                v_scale=vsd, sinks=skd, window=window)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    need = lib.sna_prefill_workspace_bytes(R, longest, H, G, d, P, width, window)
+    blocks = -(-longest // (128 // (H // G)))
+    slots = (need - 8 * G * R * blocks) // (128 * (d + 2) * 4)
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(qd)
+    rc = lib.sna_prefill_attention_split(
+        ptr(qd), ptr(kc), ptr(vc), ptr(ksd), ptr(vsd), ptr(td), td.stride(0), width, ptr(sd), ptr(pd), R, longest, ptr(skd),
+        d ** -0.5, window, ptr(out), H, G, d, P, kc.shape[0], _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_FP8_E4M3FN, ptr(ws),
+        need, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
     torch.cuda.synchronize()
     assert_close_attn(out.cpu(), want, name)
+    counts = _splits_run(ws, slots, R, blocks, G, d)
+    for r, n in enumerate(cfg["lens"]):  # a request's query blocks have splits, no others do
+        assert bool(((counts[:, r] > 0) == (torch.arange(blocks) < -(-n // (128 // (H // G))))).all()), counts
+    assert int(counts.max()) >= most if most > 1 else int(counts.max()) == 1, counts
+    packed = ops.prefill_attention(qd, kc, vc, td, sd, pd, max_q_len=longest, sm_scale=d ** -0.5, k_scale=ksd, v_scale=vsd,
+                                   sinks=skd, window=window)
+    assert torch.equal(packed, out)
     whole = _unsplit(qd, kc, vc, ksd, vsd, td, sd, pd, longest, d ** -0.5, window, skd)
     torch.cuda.synchronize()
     assert_close_attn(whole.cpu(), want, f"{name} unsplit")
-
-
-def _unsplit(q, kc, vc, ks, vs, table, q_start, priors, longest, scale, window=0, sinks=None):
-    """sna_prefill_attention: the entry without a workspace, which never splits. Device tensors."""
-    lib = _lib.load()
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    out = torch.empty_like(q)
-    rc = lib.sna_prefill_attention(ptr(q), ptr(kc), ptr(vc), ptr(ks), ptr(vs), ptr(table), table.stride(0), table.shape[1],
-                                   ptr(q_start), ptr(priors), priors.numel(), longest, ptr(sinks), scale, window, ptr(out),
-                                   q.shape[1], kc.shape[1], q.shape[2], kc.shape[2], kc.shape[0],
-                                   _lib.DTYPE_BF16 if ks is None else _lib.DTYPE_FP8_E4M3FN,
-                                   torch.cuda.current_stream().cuda_stream)
-    assert rc == 0, _lib.last_error()
-    return out
 
 
 @pytest.mark.parametrize("bf16", [False, True], ids=["fp8", "bf16"])
