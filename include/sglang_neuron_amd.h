@@ -468,8 +468,8 @@ int sna_indexer_scores(const void *q, const float *w, const uint8_t *keys, const
  * out_stride) = their positions e, those above the k-th largest value first, then its ties (the lowest positions),
  * each group in position order; a selected score <= -1e30 / 2 (a dead key) is written as -1. Exact: the selected
  * values are the k largest. B <= 65535. workspace: device memory of at least sna_topk_workspace_bytes(B, width)
- * bytes, 4-byte aligned, any contents (every word is written before it is read); calls that share a workspace on
- * different streams race.
+ * bytes, 4-byte aligned, any contents (every word is written before it is read; rows of up to 16384 scores do not touch
+ * it); calls that share a workspace on different streams race.
  * Replaces: indexer_topk_local_torch_ref's selection (indexer_torch.py:296-309); its slot order is a Trainium
  * layout, the set is the same. */
 int64_t sna_topk_workspace_bytes(int32_t B, int32_t width);

@@ -249,7 +249,7 @@ __device__ __forceinline__ uint32_t key_bits(uint32_t key) { return (key & 0x800
 //   topk_write:    the threshold key T (the k-th largest) and the count above it; positions in order: keys above T at
 //                  the running count of those before them (earlier segments' from their histograms), then T's ties
 //                  at n_above + their running count, while that is below k.
-// Workspace per row: (2 * 256 + 1) * S + 4 u32, S = ceil(width / kTopkSeg) (the last S + 4 unused).
+// Workspace per row: 2 * 256 * S u32, S = ceil(width / kTopkSeg).
 constexpr int kTopkSeg = 8192, kTopkCopies = 32, kTopkRowVecs = 2;
 
 struct TopkRow {
@@ -260,7 +260,7 @@ struct TopkRow {
 
 __device__ __forceinline__ TopkRow topk_row(const uint16_t* scores, int64_t score_stride, uint32_t* ws, int32_t S) {
   const int32_t b = blockIdx.y;
-  uint32_t* base = ws + (int64_t)b * ((2 * 256 + 1) * (int64_t)S + 4);
+  uint32_t* base = ws + (int64_t)b * (2 * 256 * (int64_t)S);
   return {scores + (int64_t)b * score_stride, base, base + 256 * S};
 }
 
@@ -577,7 +577,7 @@ int sna_indexer_scores(const void* q, const float* w, const uint8_t* keys, const
 int64_t sna_topk_workspace_bytes(int32_t B, int32_t width) {
   if (B <= 0 || width <= 0) return 0;
   const int64_t S = ((int64_t)width + kTopkSeg - 1) / kTopkSeg;
-  return (int64_t)B * ((2 * 256 + 1) * S + 4) * (int64_t)sizeof(uint32_t);
+  return (int64_t)B * 2 * 256 * S * (int64_t)sizeof(uint32_t);
 }
 
 int sna_topk_positions(const void* scores, int64_t score_stride, int32_t B, int32_t width, int32_t k, int32_t* out,

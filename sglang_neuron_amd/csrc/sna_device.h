@@ -227,7 +227,7 @@ __device__ __forceinline__ uint2 lds_read_tr16(const uint8_t* p) {
 // need. The buffer forms read through a buffer resource (a uniform base and size in SGPRs, a 32-bit offset per lane;
 // reads past the size return zeros). The LDS address is wave-uniform (readfirstlane keeps it in an SGPR for m0); the
 // s_nop covers the m0 write -> LDS-DMA hazard. The 16-byte forms carry the pool's pages, read once per decode: they
-// are non-temporal (nt), which measured ~5% faster on the MLA gathers. The _cached forms are for pages that other
+// are non-temporal (nt), which measured ~5% faster on the MLA gathers. The _cached form is for pages that other
 // workgroups read again soon (prefill: every query block of a request reads the same keys), kept in the L2.
 typedef __attribute__((address_space(3))) void lds_ptr_t;
 __device__ __forceinline__ uint32_t lds_address(const lds_ptr_t* p) {
@@ -247,16 +247,7 @@ __device__ __forceinline__ void dma_global16(const void* src, uint32_t lds) {
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m0), "v"(src) : "memory");
 }
-__device__ __forceinline__ void dma_buffer16_cached(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m0), "v"(voff), "s"(r)
-               : "memory");
-}
-__device__ __forceinline__ void dma_global16_cached(const void* src, uint32_t lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src) : "memory");
-}
-// The same with a uniform 64-bit base (SGPRs) and a 32-bit byte offset per lane, so a page's address stays scalar work.
+// From a uniform 64-bit base (SGPRs) and a 32-bit byte offset per lane, so a page's address stays scalar work.
 // (s_nop 4: a base written by a lane read just before needs five wait states until a memory instruction reads it, which
 // the compiler does not add inside an asm block.)
 __device__ __forceinline__ void dma_saddr16_cached(const void* base, uint32_t voff, uint32_t lds) {
@@ -276,29 +267,10 @@ __device__ __forceinline__ uint32_t xcd_order(uint32_t i, uint32_t n) {
   const uint32_t per = n / 8, extra = n % 8, xcd = i % 8;
   return (xcd < extra ? xcd * (per + 1) : extra * (per + 1) + (xcd - extra) * per) + i / 8;
 }
-// Lane `src`'s 64-bit value (uniform), as two lane reads.
-__device__ __forceinline__ int64_t readlane_i64(int64_t v, int src) {
-  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)(uint64_t)v, src);
-  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)v >> 32), src);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// 4x4 byte transpose with v_perm_b32 (its 8 source bytes are {S1 bytes 0-3, S0 bytes 0-3} for selector values 0-7):
-// byte r of w[e] becomes byte e of x[r].
-__device__ __forceinline__ void transpose4x4_bytes(const uint32_t (&w)[4], uint32_t (&x)[4]) {
-  const uint32_t t01l = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);  // w0.b0 w1.b0 w0.b1 w1.b1
-  const uint32_t t01h = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);  // w0.b2 w1.b2 w0.b3 w1.b3
-  const uint32_t t23l = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-  const uint32_t t23h = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-  x[0] = __builtin_amdgcn_perm(t23l, t01l, 0x05040100u);
-  x[1] = __builtin_amdgcn_perm(t23l, t01l, 0x07060302u);
-  x[2] = __builtin_amdgcn_perm(t23h, t01h, 0x05040100u);
-  x[3] = __builtin_amdgcn_perm(t23h, t01h, 0x07060302u);
 }
 
 // Two floats to a packed pair of bf16 (round to nearest even), low half first.
@@ -362,10 +334,9 @@ __device__ __forceinline__ T ld_const(const T* p) {
   return *(const __attribute__((address_space(4))) T*)(p);
 }
 
-// 16-, 8- and 4-byte global loads of raw bits.
+// 16- and 8-byte global loads of raw bits.
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ uint2 ld8(const void* p) { return *reinterpret_cast<const uint2*>(p); }
-__device__ __forceinline__ uint32_t ld4(const void* p) { return *reinterpret_cast<const uint32_t*>(p); }
 // Loads of data read once (the KV pool's pages): non-temporal, so they do not displace what the caches hold for reuse
 // (measured ~8% more HBM throughput on the paged gathers).
 __device__ __forceinline__ uint4 ld16_stream(const void* p) {
@@ -535,22 +506,6 @@ __device__ __forceinline__ void locate_work(const int32_t* __restrict__ seq_lens
     }
     base += total;
   }
-}
-
-// First flattened work index of sequence b (same decomposition), computed by one wave.
-template <int TILE>
-__device__ __forceinline__ int32_t work_base_of(const int32_t* __restrict__ seq_lens, int32_t b, int32_t window,
-                                                int32_t split_tiles) {
-  const int lane = threadIdx.x & 63;
-  int32_t acc = 0;
-  for (int32_t b0 = 0; b0 < b; b0 += 64) {
-    int32_t bb = b0 + lane;
-    int32_t n = bb < b ? splits_of<TILE>(seq_lens[bb], window, split_tiles) : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-    acc += n;
-  }
-  return acc;
 }
 
 }  // namespace sna
