@@ -13,8 +13,9 @@
 //
 // Where the query blocks alone leave CUs idle (a short chunk after a long prior) the keys are split on the device
 // (prefill_item) and a second launch merges the partials: two turns of 150 and 251 tokens after 9000 and 17000 (32 / 8
-// heads, bf16) 326 us whole, 128 split (512 workgroups; 152 with 384, 228 with 256); 16 tokens after 30000 (FP8) 478 and
-// 53; 64 after 3000, 59 and 31.
+// heads, bf16) 322 us whole, 116 split (512 workgroups; with 384 and 256 a fifth and four fifths longer); 16 tokens after
+// 30000 (FP8) 469 and 47; 64 after 3000, 56 and 26. The search and the merge launch cost 5-6 us where the device's
+// lengths leave nothing to split (8 requests of 100 tokens after 4000, bf16: 84 us unsplit, 90 here).
 //
 // Lane roles (lane = 32 g2 + i), per sub-tile of 32 keys:
 //   QK  S^T[key, row] = K[key, :] . Q[row, :]: lane (g2, i) feeds A row i, the key whose index swaps bits 2 and 3 of i.
@@ -31,12 +32,12 @@
 //
 // What bounds it: the matrix cores under the card's power limit. On four requests of 2048 tokens after 2048 (32 / 8
 // heads of 128, FP8) the clock settles near 1.87 GHz and the matrix pipe is busy 57% of the cycles; without the QK
-// products the launch takes 278 us, without PV's 316, without the exponentials 348, against 377-384 us (1.07-1.09
-// PFLOP/s; a large bf16 GEMM reaches 1.38 on the same card). Steps of this form, from 432 us: whole-row swizzled DMAs
-// and masks only in boundary tiles (VALU per tile and wave 307 -> 205) 388; the 32 x 32 shapes 388 (half the matrix
-// instructions, the same time); the next tile's QK beside this tile's softmax 380. bf16 pools, the same batch: 571 ->
-// 418 us, V^T straight from the ring instead of through a shared bf16 copy. Head dim 64 (8 heads on one, FP8, sinks):
-// 112 -> 93 us.
+// products the launch took 278 us, without PV's 316, without the exponentials 348, against 380 us then; alone in graph
+// replays it takes 350-366 us (1.13-1.18 PFLOP/s; a large bf16 GEMM reaches 1.38 on the same card). Steps of this form,
+// from 432 us: whole-row swizzled DMAs and masks only in boundary tiles (VALU per tile and wave 307 -> 205) 388; the 32
+// x 32 shapes 388 (half the matrix instructions, the same time); the next tile's QK beside this tile's softmax 380. bf16
+// pools, the same batch: 571 -> 418 us (now 400-417), V^T straight from the ring instead of through a shared bf16 copy.
+// Head dim 64 (8 heads on one, FP8, sinks): 112 -> 93 us.
 
 #include <algorithm>
 #include <type_traits>
@@ -135,10 +136,10 @@ __device__ __forceinline__ PrefillBlock prefill_block(const PrefillArgs& a, int3
 // The item w of a workgroup of a launch that splits the keys. Every (request, query block, KV head) is cut into splits
 // of st tiles, st the least size (at least min_tiles) whose items fit the launch's workgroups; the pairs' tile counts
 // come from the device's lengths, 4 a lane in registers, and every wave computes the same st and item. The split is
-// dropped (st the longest block) where it would not pay: a tile takes about 1.3 us up to one workgroup a CU and 2 us
-// with two (the card's power limit holds the chip to some 270 tiles a microsecond), the partials of 32 items 1 us of the
-// launch and the merge pass 5 us. w numbers the items KV head by KV head, then pair by pair (request-major), a pair's
-// splits in order. Every lane gets the same values; false past the last item.
+// dropped (st the longest block) where it would not pay (fitted at head dim 128 and 256 CUs): a tile takes about 1.3 us
+// up to one workgroup a CU and 2 us with two (the card's power limit holds the chip to some 270 tiles a microsecond),
+// the partials of 32 items 1 us of the launch and the merge pass 5 us. w numbers the items KV head by KV head, then pair
+// by pair (request-major), a pair's splits in order. Every lane gets the same values; false past the last item.
 __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32_t& r, int32_t& bx, int32_t& split,
                              int32_t& st_out, int32_t& ns) {
   constexpr int N = kPrefillSplitPairs / 64;
@@ -232,10 +233,10 @@ __device__ bool prefill_item(const PrefillArgs& a, int32_t& w, int32_t& g, int32
   return found;
 }
 
-// kOneTile and kHalfTile: the launch's tables name at most one tile of keys, or 32 of them (prompts of up to 64 or 32 tokens
-// with no prior), so the loop's next tile, whose products it computes whether there is one or not, and the tile's second
-// sub-tile are left out (32 / 8 heads of 128, FP8 / bf16, us: 16 tokens 8.2 / 7.6 through the loop, 6.9 / 6.2 so; 60 tokens 9.0 /
-// 8.4 and 8.7 / 8.0; as runtime branches of one kernel 7.8 / 7.4 and 9.1 / 9.0).
+// kOneTile and kHalfTile: the launch's tables name at most one tile of keys, or 32 of them (prompts of up to 64 or 32
+// tokens with no prior), so the loop's next tile, whose products it computes whether there is one or not, and the tile's
+// second sub-tile are left out (32 / 8 heads of 128, FP8 / bf16, us: 16 tokens 8.2 / 7.6 through the loop, 6.9 / 6.2 so;
+// 60 tokens 9.0 / 8.4 and 8.7 / 8.0; as runtime branches of one kernel 7.8 / 7.4 and 9.1 / 9.0).
 enum PrefillMode { kWhole, kSplit, kOneTile, kHalfTile };
 template <int D, int ESZ, PrefillMode MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
@@ -255,14 +256,14 @@ void prefill_gqa_kernel(PrefillArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63, g2 = lane >> 5, i32 = lane & 31, li = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int32_t bx, r, g, split = 0, split_tiles = 0, ns = 1, item = 0;
+  int32_t bx, r, g, split = 0, split_tiles = 0, ns = 1, item = 0, note = -1;
   if constexpr (SPLIT) {
     // the same in every lane: made scalar, so what is addressed with them stays in scalar registers
     if (!__builtin_amdgcn_readfirstlane((int)prefill_item(a, item, g, r, bx, split, split_tiles, ns))) return;
     g = __builtin_amdgcn_readfirstlane(g), r = __builtin_amdgcn_readfirstlane(r);
     bx = __builtin_amdgcn_readfirstlane(bx), split = __builtin_amdgcn_readfirstlane(split);
     split_tiles = __builtin_amdgcn_readfirstlane(split_tiles), ns = __builtin_amdgcn_readfirstlane(ns);
-    if (split == 0 && tid == 0) a.ws_item[((int64_t)g * a.R + r) * a.qblocks + bx] = make_int2(item, ns);
+    if (split == 0) note = (g * a.R + r) * a.qblocks + bx;  // (ws_item's entry of the block)
   } else {
     // XCD-aware order: each XCD takes a contiguous run of the (query block, request, KV head) order, so the query
     // blocks that read the same request's keys of one KV head share that XCD's L2
@@ -611,6 +612,15 @@ void prefill_gqa_kernel(PrefillArgs a) {
   int32_t row = 32 * wave + i32;
   asm volatile("" : "+v"(row));
   const bool row_ok = token_of(row) < nq;
+  // Of a launch that splits, a block's first item and split count, written by the thread of its first row (always valid).
+  // Last, and by an index made at the head: with a store to memory before the loop the compiler no longer takes the
+  // lengths, scales and tables for unchanging, and with the block's three indices held over the loop it runs out of
+  // registers; either way the loop waits for every LDS read by itself (a turn of 128-dim rows 1.1 times the unsplit
+  // kernel's with FP8 and 1.35 times with bf16 pools: 8 requests of 100 tokens after 4000, 32 / 8 heads, 86 and 113 us,
+  // so 80 and 90).
+  auto note_item = [&]() {
+    if (SPLIT && note >= 0 && tid == 0) a.ws_item[note] = make_int2(item, ns);
+  };
   if (SPLIT && ns > 1) {  // this split's partial: the combine pass merges the block's splits
     if (!row_ok) return;
     float* wo = a.ws_o + ((int64_t)item * kPrefillRows + row) * D + 4 * g2;
@@ -622,6 +632,7 @@ void prefill_gqa_kernel(PrefillArgs a) {
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4_t*>(wo + 32 * c + 8 * q) =
             f32x4_t{acc[c][4 * q], acc[c][4 * q + 1], acc[c][4 * q + 2], acc[c][4 * q + 3]};
+    note_item();
     return;
   }
   // ---- epilogue: normalize (sinks join the denominator), scale by v_scale, write the valid rows ----
@@ -636,10 +647,11 @@ void prefill_gqa_kernel(PrefillArgs a) {
       *reinterpret_cast<uint2*>(dst + 32 * c + 8 * q) =
           make_uint2(pack_bf16x2(acc[c][4 * q] * inv, acc[c][4 * q + 1] * inv),
                      pack_bf16x2(acc[c][4 * q + 2] * inv, acc[c][4 * q + 3] * inv));
+  note_item();
 }
 
-// Merge of the split query blocks, 1024 / D of a block's rows a workgroup: out = sum_s e_s o_s / (sum_s e_s l_s + e_sink) with
-// e_s = exp2(m_s - M), M the largest m_s. D / 4 lanes a row, the loads of four splits in flight together.
+// Merge of the split query blocks, 1024 / D of a block's rows a workgroup: out = sum_s e_s o_s / (sum_s e_s l_s +
+// e_sink) with e_s = exp2(m_s - M), M the largest m_s. D / 4 lanes a row, the loads of four splits in flight together.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a, bool fp8) {
   constexpr int LR = D / 4;  // lanes a row
@@ -684,8 +696,9 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a, boo
 }
 
 // The workgroups of a split launch: 0 where the launch's own query blocks are more than one a CU (they reach the rate
-// that the power limit allows by themselves: 352 blocks of up to 137 tiles took 170 us whole, 186 in a split launch; 376
-// of up to 24 tiles 41 and 49), too short, or past what the split counts.
+// that the power limit allows by themselves: 352 blocks of up to 136 tiles took 201 us whole, 206 in a split launch; 376
+// of up to 24 tiles 36 and 42; requests of unequal lengths would gain, which the host does not know), too short (the
+// search and the merge launch), or past what the split counts.
 static int32_t prefill_split_slots(int64_t qblocks, int32_t R, int32_t G, int64_t bound_tiles) {
   const int64_t base = qblocks * R * G;
   if (base > kPrefillSplitBlocks || bound_tiles <= kPrefillNoSplit || bound_tiles > kPrefillSplitMaxTiles) return 0;
