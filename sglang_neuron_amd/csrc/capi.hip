@@ -317,9 +317,9 @@ int sna_plan_decode(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32
   plan->max_splits = max_splits;
   plan->batch = B;
   if (kind == 0 && !host_seq_lens && B <= kGqaDevSplitRows && bound_tiles <= kGqaDevSplitMaxTiles) {
-    // A GQA plan from a bound splits on the device: every launch sizes its splits from the device's lengths by the
-    // one-round rule above to fit the items the bound's own split runs, and gives every row a split (a row with no
-    // prior key attends its own token there: no lone-token pass). A split holds at least 4 tiles and at least
+    // A GQA plan from a bound splits on the device: every launch sizes its splits from the device's lengths by a
+    // one-round rule (rows of up to 8 tiles whole) to fit the items the bound's own split runs, and gives every row a
+    // split (a row with no prior key attends its own token there: no lone-token pass). A split holds at least 4 tiles and at least
     // min(longest row, 8), so a row of up to 8 tiles is one split and a longer one at most ceil(tiles / 8); and as
     // every other row takes an item, a row gets at most n_work - B + 1 (one, when the bound's split is whole rows).
     plan->device_split = 1;

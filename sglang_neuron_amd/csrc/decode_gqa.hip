@@ -90,9 +90,9 @@ __device__ __forceinline__ int32_t launched_splits(const GqaArgs& a, int32_t b, 
 
 // A device split's item (every lane of the calling wave gets the same values): the launch's split size st and, for
 // item w, its row b (-1 past the last item), split and the row's seq_len L, from one load of every row's length.
-// Every row has at least one split (launched_splits). The split size is the host planner's one-round rule applied
-// to the device's lengths: at least 4 tiles and ceil(total tiles / items), at least min(longest row, 8) tiles, at
-// most the longest row, grown to the least size whose items (sum over rows of max(1, ceil(tiles / size))) fit the
+// Every row has at least one split (launched_splits). The split size is a one-round rule on the device's lengths, the
+// host planner's but for the rows it keeps whole (up to 8 tiles here, up to 12 or 24 in a plan of exact lengths): at
+// least 4 tiles and ceil(total tiles / items), at least min(longest row, 8) tiles, at most the longest row, grown to the least size whose items (sum over rows of max(1, ceil(tiles / size))) fit the
 // launch's n_work, and at least a 64th of the longest row (a row's splits fit the combine's 64 weights). The least
 // size is bisected between that start and ceil(total / (items - B)), which fits (each row's count is below
 // tiles / size + 1). The rows' lengths and tile counts stay in registers: B <= kGqaDevSplitRows, n_work >= B (so the

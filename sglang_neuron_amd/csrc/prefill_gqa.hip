@@ -33,7 +33,7 @@
 // What bounds it: the matrix cores under the card's power limit. On four requests of 2048 tokens after 2048 (32 / 8
 // heads of 128, FP8) the clock settles near 1.87 GHz and the matrix pipe is busy 57% of the cycles; without the QK
 // products the launch took 278 us, without PV's 316, without the exponentials 348, against 380 us then; alone in graph
-// replays it takes 350-366 us (1.13-1.18 PFLOP/s; a large bf16 GEMM reaches 1.38 on the same card). Steps of this form,
+// replays it takes 350-380 us (1.09-1.18 PFLOP/s; a large bf16 GEMM reaches 1.38 on the same card). Steps of this form,
 // from 432 us: whole-row swizzled DMAs and masks only in boundary tiles (VALU per tile and wave 307 -> 205) 388; the 32
 // x 32 shapes 388 (half the matrix instructions, the same time); the next tile's QK beside this tile's softmax 380. bf16
 // pools, the same batch: 571 -> 418 us (now 400-417), V^T straight from the ring instead of through a shared bf16 copy.
