@@ -430,7 +430,8 @@ int sna_prefill_attention(const void *q, const void *k_cache, const void *v_cach
  * query block's keys are cut on the device, from its lengths, into splits that fill one or two rounds of workgroups, the
  * partials go to `workspace` (device, 16-byte aligned, at least sna_prefill_workspace_bytes bytes; it needs no
  * initialisation) and a second launch merges them. A NULL workspace never splits. sna_prefill_workspace_bytes: 0 where
- * the launch would not split. */
+ * the launch would not split. That goes by max_q_len and the table's width, the lengths being on the device: a table
+ * much wider than the batch's pages costs a short batch the search and the merge launch (2-6 us). */
 int64_t sna_prefill_workspace_bytes(int32_t R, int32_t max_q_len, int32_t num_q_heads, int32_t num_kv_heads,
                                     int32_t head_dim, int32_t page_size, int32_t table_width, int32_t window);
 int sna_prefill_attention_split(const void *q, const void *k_cache, const void *v_cache, const float *k_scale,

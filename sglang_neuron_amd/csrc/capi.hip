@@ -272,8 +272,10 @@ int sna_plan_decode(int32_t kind, const int32_t* host_seq_lens, int32_t B, int32
   int32_t split_tiles = (int32_t)std::max<int64_t>(waves, (total_tiles + items_target - 1) / items_target);
   // short rows (a sliding window, a few pages) stay whole: one split, no combine pass. Rows of up to 12 tiles always
   // (graph replays, 16 / 8 heads of 128, bf16: one row of 10 tiles 8.5 -> 7.7 us, eight of 12 tiles 10.0 -> 9.8; of 14,
-  // 10.3 -> 11.4), of up to 24 where the whole rows already give every CU a workgroup (32 rows of up to 24 tiles, 32 / 8
-  // heads, FP8: 16.4 -> 12.1 us; of 16 tiles, bf16, 16.8 -> 14.3)
+  // 10.3 -> 11.4), of up to 24 where the whole rows already give every CU a workgroup (rows of 24 tiles, 32 / 8 heads,
+  // FP8 and bf16, us: 32 rows 21.6 -> 11.9 and 26.9 -> 18.4, 64 rows 23.2 -> 20.7 and 35.9 -> 33.9, 128 rows 45.9 ->
+  // 37.7 and 71.3 -> 63.8, 32 ragged rows of up to 27 tiles 19.7 -> 15.4 and 24.0 -> 22.6; head dim 64, 32 rows 13.8 ->
+  // 8.7 and 17.7 -> 11.3, more rows the same)
   split_tiles = std::max(split_tiles, std::min(max_tiles, 2 * waves));
   if (max_tiles <= 12 || (max_tiles <= 24 && (int64_t)B * ctas_per_item >= cus))
     split_tiles = std::max(split_tiles, max_tiles);
